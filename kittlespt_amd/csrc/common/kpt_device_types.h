@@ -23,19 +23,24 @@ struct alignas(16) Node {
 };
 static_assert(sizeof(Node) == 32, "Node is 32 bytes");
 
-// Two BVH levels in one 192-byte record, for the traversal kernels: the
-// children pair of an interior node (c0, c1: copies of nodes 2q and 2q+1 of
-// the level's pair layout, where q is the record index) and, for each
-// interior child, its own children (g0, g1 for c0; g2, g3 for c1; zero
-// otherwise).  BLAS records follow the BLAS node array (sibling pairs at even
-// indices); TLAS records follow a renumbered copy of the TLAS in the same
-// pair layout (root at 0, pairs from 2 on; interior a = children pair index,
-// leaf a = 0, b = instance).
-struct alignas(64) NodeBlock {
-    Node c[2];
-    Node g[4];
+// The children of one interior node as the traversal reads them, one 64-byte
+// line: both boxes and, in place of the nodes' header words, each child's
+// traversal entry (kpt_trace.h).  One array holds both levels: the TLAS's
+// pairs first (num_instances + 1 records, from a renumbered copy of the TLAS
+// in the pair layout: root at 0, pairs from 2 on; interior a = children pair
+// index, leaf a = 0, b = instance), then the BLAS's (sibling pairs at even
+// node indices), record q of a level being its nodes 2q and 2q + 1.
+struct alignas(64) NodePair {
+    float lo0[3];
+    uint32_t e0;
+    float hi0[3];
+    uint32_t pad0;
+    float lo1[3];
+    uint32_t e1;
+    float hi1[3];
+    uint32_t pad1;
 };
-static_assert(sizeof(NodeBlock) == 192, "NodeBlock is 192 bytes");
+static_assert(sizeof(NodePair) == 64, "NodePair is 64 bytes");
 
 // Triangle positions in BVH-leaf (slot) order: v0 and the two edges the
 // Moller-Trumbore test needs (triangle.cuh:66-102 computes v1-v0 and v2-v0 per
@@ -152,9 +157,8 @@ struct alignas(16) FrameConst {
 // Scene pointers passed by value to kernels.
 struct SceneView {
     const Node* blas_nodes;
-    const Node* tlas_nodes;      // pair layout (see NodeBlock)
-    const NodeBlock* blas_blocks;
-    const NodeBlock* tlas_blocks;
+    const Node* tlas_nodes;      // pair layout (see NodePair)
+    const NodePair* pairs;       // TLAS pairs, then BLAS pairs
     const TriPos* tris;
     const TriAttr* attrs;
     const InstTrav* inst_trav;

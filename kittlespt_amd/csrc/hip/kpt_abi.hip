@@ -81,8 +81,8 @@ struct kpt_ctx {
     // device scene
     Node* d_blas = nullptr;
     Node* d_tlas = nullptr;          // TLAS in the pair layout of the traversal
-    NodeBlock* d_bblocks = nullptr;  // two-level records of the BLAS pairs
-    NodeBlock* d_tblocks = nullptr;  // two-level records of the TLAS pairs
+    NodePair* d_pairs = nullptr;     // the traversal's pairs: first_pair TLAS records, then the BLAS's
+    uint32_t first_pair = 0;         // num_instances + 1
     TriPos* d_tris = nullptr;
     TriAttr* d_attrs = nullptr;
     InstTrav* d_itrav = nullptr;
@@ -194,8 +194,7 @@ SceneView scene_view(const kpt_ctx* c) {
     SceneView S;
     S.blas_nodes = c->d_blas;
     S.tlas_nodes = c->d_tlas;
-    S.blas_blocks = c->d_bblocks;
-    S.tlas_blocks = c->d_tblocks;
+    S.pairs = c->d_pairs;
     S.tris = c->d_tris;
     S.attrs = c->d_attrs;
     S.inst_trav = c->d_itrav;
@@ -213,29 +212,23 @@ SceneView scene_view(const kpt_ctx* c) {
 
 void store_mat(const hm::Mat4& m, float* dst) { std::memcpy(dst, m.m, 64); }
 
-// Two-level records of a pair-layout node array (see NodeBlock): record q
-// holds nodes 2q, 2q+1 and the children of each interior one.  `interior`
-// tells the level's interior test; `pair` gives an interior node's children
-// pair index.  Returns false when a children pair does not sit at an even
-// index (the layout the traversal relies on).
-template <class IsInterior>
-bool make_blocks(const std::vector<Node>& nodes, IsInterior interior, std::vector<NodeBlock>* out) {
-    out->assign(nodes.size() / 2 + 1, NodeBlock{});
-    for (size_t i = 0; i < nodes.size(); ++i) {
-        const Node& x = nodes[i];
-        if (!interior(x)) continue;
-        const uint32_t p = x.a;
-        if ((p & 1u) || (size_t)p + 1 >= nodes.size()) return false;
-        NodeBlock& blk = (*out)[p >> 1];
-        blk.c[0] = nodes[p];
-        blk.c[1] = nodes[p + 1];
-        for (int k = 0; k < 2; ++k) {
-            const Node& ch = nodes[p + k];
-            if (!interior(ch)) continue;
-            if ((ch.a & 1u) || (size_t)ch.a + 1 >= nodes.size()) return false;
-            blk.g[2 * k] = nodes[ch.a];
-            blk.g[2 * k + 1] = nodes[ch.a + 1];
-        }
+// The TLAS's pairs (see NodePair) from its pair layout: one record per merged
+// node, the first and the last left empty.
+std::vector<NodePair> tlas_pairs(const std::vector<Node>& nodes) {
+    std::vector<NodePair> out(nodes.size() / 2 + 1, NodePair{});
+    for (size_t q = 1; 2 * q + 1 < nodes.size(); ++q) out[q] = tlas_pair(nodes[2 * q], nodes[2 * q + 1]);
+    return out;
+}
+
+// The BLAS's pairs from the global node array.  Returns false when an
+// interior node's children do not sit at an even index and the next one (the
+// layout the traversal relies on).
+bool blas_pairs(const std::vector<Node>& nodes, uint32_t first_pair, std::vector<NodePair>* out) {
+    out->assign(nodes.size() / 2 + 1, NodePair{});
+    for (const Node& x : nodes) {
+        if (x.b != 0u || x.a == 0u) continue;   // a leaf, or a padding node
+        if ((x.a & 1u) || (size_t)x.a + 1 >= nodes.size()) return false;
+        (*out)[x.a >> 1] = blas_pair(nodes[x.a], nodes[x.a + 1], x.a >> 1, first_pair);
     }
     return true;
 }
@@ -278,10 +271,10 @@ void make_instance(kpt_ctx* c, int32_t i, const float* model, bool keep_prev) {
     int32_t g = c->inst_mesh[i];
     it.root = c->blas[g].used > 0 ? c->geom_base[g] : -1;
     it.geom = g;
-    it.root_entry = 0xFFFFFFFFu;
+    it.root_entry = ENTRY_IDLE;
     if (it.root >= 0) {
         const Node& r = c->nodes[(size_t)it.root];
-        it.root_entry = blas_entry((uint32_t)it.root, r.a, r.b);
+        it.root_entry = blas_entry((uint32_t)it.root, r.a, r.b, c->first_pair);
     }
     InstShade& sh = c->ishade[i];
     hm::Mat4 curr_inv = hm::glm_inverse(M);
@@ -311,9 +304,9 @@ int upload_tlas(kpt_ctx* ctx) {
     if (ctx->tlas.nodes.size() > 65535) return fail(ctx, KPT_ERR_UNSUPPORTED, "TLAS exceeds 65535 nodes (16-bit child fields)");
     if (ctx->host_only) return KPT_OK;
     const std::vector<Node> tp = tlas_pair_layout(ctx->tlas.nodes);
-    std::vector<NodeBlock> tb;
-    if (!make_blocks(tp, [](const Node& n) { return n.a != 0u; }, &tb))
-        return fail(ctx, KPT_ERR_UNSUPPORTED, "TLAS pair layout failed");
+    const std::vector<NodePair> tb = tlas_pairs(tp);
+    if (tb.size() > (size_t)ctx->first_pair || !ctx->d_pairs)
+        return fail(ctx, KPT_ERR_STATE, "TLAS larger than its place in the pair array");
     // the previous frame may still read the old arrays
     HIPCHK(hipStreamSynchronize(ctx->stream));
     // the device rebuild's buffers follow the instance count of this tree
@@ -323,7 +316,7 @@ int upload_tlas(kpt_ctx* ctx) {
     dev_free(&ctx->d_tlas_parent);
     dev_free(&ctx->d_tlas_arrivals);
     HIPCHK(dev_upload(&ctx->d_tlas, tp));
-    HIPCHK(dev_upload(&ctx->d_tblocks, tb));
+    HIPCHK(hipMemcpy(ctx->d_pairs, tb.data(), tb.size() * sizeof(NodePair), hipMemcpyHostToDevice));
     HIPCHK(dev_upload(&ctx->d_itrav, ctx->itrav));
     HIPCHK(dev_upload(&ctx->d_ishade, ctx->ishade));
     if (ctx->tlas_device == 2 && !ctx->tlas.nodes.empty()) {
@@ -354,7 +347,7 @@ int rebuild_tlas_device(kpt_ctx* ctx) {
     const int32_t N = (int32_t)ctx->inst_bounds.size();
     const bool refit = ctx->tlas_device == 2;
     bool ok = ctx->tlas_device && !ctx->host_only && N >= 1 && (refit || N <= TLAS_DEVICE_MAX) &&
-              ctx->d_tlas && ctx->d_tblocks && (int64_t)ctx->tlas.nodes.size() == 2 * (int64_t)N &&
+              ctx->d_tlas && ctx->d_pairs && (int64_t)ctx->tlas.nodes.size() == 2 * (int64_t)N &&
               (!refit || (ctx->d_tlas_parent && ctx->d_tlas_ref));
     for (int32_t i = 0; ok && i < N; ++i)
         for (int k = 0; k < 3; ++k) {
@@ -371,7 +364,7 @@ int rebuild_tlas_device(kpt_ctx* ctx) {
         HIPCHK(hipMemcpyAsync(ctx->d_ishade, ctx->ishade.data(), ctx->ishade.size() * sizeof(InstShade),
                               hipMemcpyHostToDevice, ctx->stream));
         HIPCHK(launch_tlas_refit(ctx->stream, ctx->d_inst_bounds, N, ctx->d_tlas_ref, ctx->d_tlas_parent,
-                                 ctx->d_tlas_arrivals, ctx->d_tlas, ctx->d_tblocks, ctx->d_tlas_status));
+                                 ctx->d_tlas_arrivals, ctx->d_tlas, ctx->d_pairs, ctx->d_tlas_status));
         ctx->tlas_dirty = false;
         ctx->tlas_on_device = true;
         set_scene_box(ctx);
@@ -389,7 +382,7 @@ int rebuild_tlas_device(kpt_ctx* ctx) {
                           hipMemcpyHostToDevice, ctx->stream));
     HIPCHK(hipMemcpyAsync(ctx->d_ishade, ctx->ishade.data(), ctx->ishade.size() * sizeof(InstShade),
                           hipMemcpyHostToDevice, ctx->stream));
-    HIPCHK(launch_tlas_build(ctx->stream, ctx->d_inst_bounds, N, ctx->d_tlas_ref, ctx->d_tlas, ctx->d_tblocks,
+    HIPCHK(launch_tlas_build(ctx->stream, ctx->d_inst_bounds, N, ctx->d_tlas_ref, ctx->d_tlas, ctx->d_pairs,
                              ctx->d_tlas_status));
     ctx->tlas_dirty = false;
     ctx->tlas_on_device = true;
@@ -798,7 +791,7 @@ int kpt_ctx_destroy(kpt_ctx* ctx) {
             if (ctx->lane_done[k]) (void)hipEventDestroy(ctx->lane_done[k]);
         if (ctx->stream2) (void)hipStreamDestroy(ctx->stream2);
         dev_free(&ctx->d_blas); dev_free(&ctx->d_tlas); dev_free(&ctx->d_tris); dev_free(&ctx->d_attrs);
-        dev_free(&ctx->d_bblocks); dev_free(&ctx->d_tblocks);
+        dev_free(&ctx->d_pairs);
         dev_free(&ctx->d_itrav); dev_free(&ctx->d_ishade); dev_free(&ctx->d_mat); dev_free(&ctx->d_tex);
         dev_free(&ctx->d_pix); dev_free(&ctx->d_lights); dev_free(&ctx->d_lverts); dev_free(&ctx->d_overflow);
         free_frame(ctx);
@@ -1030,6 +1023,7 @@ int kpt_upload_scene(kpt_ctx* ctx, const kpt_scene_desc* d) {
         }
     }
     // instances + TLAS
+    ctx->first_pair = (uint32_t)NI + 1u;
     ctx->itrav.assign(NI, InstTrav());
     ctx->ishade.assign(NI, InstShade());
     ctx->inst_bounds.assign(NI, Aabb());
@@ -1037,12 +1031,16 @@ int kpt_upload_scene(kpt_ctx* ctx, const kpt_scene_desc* d) {
     if (!ctx->host_only) {
         HIPCHK(hipSetDevice(ctx->device));
         HIPCHK(dev_upload(&ctx->d_blas, ctx->nodes));
-        std::vector<NodeBlock> bb;
-        if (!make_blocks(ctx->nodes, [](const Node& n) { return n.b == 0u; }, &bb))
+        std::vector<NodePair> bp;
+        if (!blas_pairs(ctx->nodes, ctx->first_pair, &bp))
             return fail(ctx, KPT_ERR_UNSUPPORTED, "BLAS sibling pair not at an even node index");
-        if (ctx->nodes.size() >= (size_t)ENTRY_PAYLOAD)
+        if (ctx->nodes.size() >= (size_t)ENTRY_PAYLOAD || ctx->first_pair + bp.size() >= (size_t)ENTRY_PAYLOAD)
             return fail(ctx, KPT_ERR_UNSUPPORTED, "BLAS node count exceeds the traversal entry range");
-        HIPCHK(dev_upload(&ctx->d_bblocks, bb));
+        // room for the TLAS's pairs (upload_tlas, the device rebuild) ahead of the BLAS's
+        dev_free(&ctx->d_pairs);
+        HIPCHK(hipMalloc((void**)&ctx->d_pairs, (ctx->first_pair + bp.size()) * sizeof(NodePair)));
+        HIPCHK(hipMemcpy(ctx->d_pairs + ctx->first_pair, bp.data(), bp.size() * sizeof(NodePair),
+                         hipMemcpyHostToDevice));
         HIPCHK(dev_upload(&ctx->d_tris, tris));
         HIPCHK(dev_upload(&ctx->d_attrs, attrs));
         HIPCHK(dev_upload(&ctx->d_mat, ctx->materials));

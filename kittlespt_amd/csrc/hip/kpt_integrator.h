@@ -43,6 +43,7 @@ struct NeeResult {
     float tmax;
     v3 unoccl;
     v3 occl;
+    int32_t trec;   // radiance cache: the training record whose radiance-so-far follows this estimate (-1: none)
 };
 
 // sampleLdSun / sampleLd and the L += Ld*beta/p of integrator.cuh:365-375,
@@ -55,6 +56,7 @@ KD NeeResult next_event(const SceneView& S, const FrameConst& fc, const Surf& s,
                         uint32_t& seed, float sun_p = 0.5f) {
     NeeResult r;
     r.trace = false;
+    r.trec = -1;
     const v3 zero = mk3(0.0f, 0.0f, 0.0f);
     if (rng1(seed) < sun_p) {
         // sampleLdSun, integrator.cuh:147-186
@@ -222,48 +224,27 @@ KD CacheVertex cache_vertex(const FrameConst& fc, const CacheBuffers& cb, const 
     return cv;
 }
 
-// One vertex of Li's loop (integrator.cuh:266-399): trace from the path's
-// ray, add emission and the next-event estimate, sample the next direction.
-// Returns false where the reference's loop breaks (miss, last depth, zero
-// BSDF sample, Russian roulette); the caller also stops when beta is zero.
+// One vertex of Li's loop (integrator.cuh:266-399) after its closest-hit trace
+// (h, from ps.ray): adds emission, samples the next-event estimate and the
+// next direction.  Returns false where the reference's loop breaks (miss, last
+// depth, zero BSDF sample, Russian roulette); the caller also stops when beta
+// is zero.  The estimate's shadow ray is left to the caller (ne->trace), who
+// traces it with the wave's others and adds its term (li_resolve) before the
+// next vertex: its answer only picks the term added to L, and nothing else
+// touches L in between.
 // DEFER_SKY (vertices past the first only): a miss sets *missed and leaves
 // L without the sky term — the last addition of the path, L + sky * beta,
 // which the caller then makes with ps.ray.d and ps.beta as they are.
 // CACHE: the radiance cache's hooks at the path's cache vertex (cache_vertex
 // with path index `path`), as the wavefront's shade stage applies them; a
 // path that ends in the network returns false after its next-event estimate.
-// heat (COUNT with cnt): the path's pixel's DebugData pair, to which the
-// closest-hit trace's BLAS and TLAS node pops are added.
-// li_shade is the vertex after its closest-hit trace (h, from ps.ray): the
-// part li_bounce and the wavefront tail share.
-template <bool COUNT = false, bool DEFER_SKY = false, bool CACHE = false>
-KD bool li_shade(const SceneView& S, const FrameConst& fc, PathState& ps, uint32_t& seed, const Hit& h,
-                 const StackShape& lds, bool* ovf, VisOut* vs, TraceCounts* cnt = nullptr, bool* missed = nullptr,
-                 const CacheBuffers* cb = nullptr, const CacheFrame* cf = nullptr, int32_t path = -1,
-                 uint32_t* spill = nullptr);
-
-template <bool COUNT = false, bool DEFER_SKY = false, bool CACHE = false>
-KD bool li_bounce(const SceneView& S, const FrameConst& fc, PathState& ps, uint32_t& seed, const StackShape& lds,
-                  bool* ovf, VisOut* vs, TraceCounts* cnt = nullptr, bool* missed = nullptr,
-                  const CacheBuffers* cb = nullptr, const CacheFrame* cf = nullptr, int32_t path = -1,
-                  int32_t* heat = nullptr) {
-    seed = seed + (uint32_t)ps.depth;
-    bool o = false;
-    const uint32_t b0 = (COUNT && cnt) ? cnt->interior + cnt->leaf : 0u, t0 = (COUNT && cnt) ? cnt->tlas : 0u;
-    Hit h = trace_closest<COUNT>(S, ps.ray, 0.0f, __builtin_inff(), lds, &o, cnt);
-    if (COUNT && cnt && heat) {
-        atomicAdd(&heat[0], (int32_t)(cnt->interior + cnt->leaf - b0));
-        atomicAdd(&heat[1], (int32_t)(cnt->tlas - t0));
-    }
-    *ovf = *ovf || o;
-    return li_shade<COUNT, DEFER_SKY, CACHE>(S, fc, ps, seed, h, lds, ovf, vs, cnt, missed, cb, cf, path);
-}
-
-template <bool COUNT, bool DEFER_SKY, bool CACHE>
-KD bool li_shade(const SceneView& S, const FrameConst& fc, PathState& ps, uint32_t& seed, const Hit& h,
-                 const StackShape& lds, bool* ovf, VisOut* vs, TraceCounts* cnt, bool* missed,
-                 const CacheBuffers* cb, const CacheFrame* cf, int32_t path, uint32_t* spill) {
+template <bool DEFER_SKY = false, bool CACHE = false>
+KD bool li_shade(const SceneView& S, const FrameConst& fc, PathState& ps, uint32_t& seed, const Hit& h, VisOut* vs,
+                 NeeResult* ne, bool* missed = nullptr, const CacheBuffers* cb = nullptr,
+                 const CacheFrame* cf = nullptr, int32_t path = -1) {
     const float eta_scale = 1.0f;
+    ne->trace = false;
+    ne->trec = -1;
     const bool first = (ps.depth == 0);
     if (DEFER_SKY && h.slot < 0 && !first) {
         *missed = true;
@@ -299,17 +280,16 @@ KD bool li_shade(const SceneView& S, const FrameConst& fc, PathState& ps, uint32
             cv.trec = -1;
         }
     }
-    // The next-event estimate's random numbers are drawn here, before the
-    // continuation's, as the reference draws them; its shadow ray is traced
-    // after the continuation is sampled (its answer only picks the term added
-    // to L, and nothing else touches L in between), so the surface and BSDF
-    // are no longer live while it runs.
-    NeeResult ne;
-    ne.trace = false;
-    bool nee = false;
+    // The next-event estimate's random numbers are drawn before the
+    // continuation's, as the reference draws them.
     if (!(CACHE && cv.to_cache && !cf->nee) && !(b.alpha < 0.001f)) {
-        ne = next_event(S, fc, s, b, ps.ray.d, ps.beta, seed, cv.sun_p);
-        nee = true;
+        *ne = next_event(S, fc, s, b, ps.ray.d, ps.beta, seed, cv.sun_p);
+        if (!ne->trace) ps.L = ps.L + ne->occl;
+    }
+    // a training record's radiance so far includes the vertex's estimate
+    if (CACHE && cv.trec >= 0) {
+        if (ne->trace) ne->trec = cv.trec;
+        else cb->t_lbefore[cv.trec] = make_float4(ps.L.x, ps.L.y, ps.L.z, 0.0f);
     }
     bool more = true;
     if (ps.depth++ == fc.max_depth) more = false;
@@ -337,37 +317,20 @@ KD bool li_shade(const SceneView& S, const FrameConst& fc, PathState& ps, uint32
             }
         }
     }
-    if (nee) {
-        if (ne.trace) {
-            bool oo = false;
-            Ray sr = make_ray(ne.org, ne.dir);
-            // the caller's stack spill area when it has one (its closest-hit trace has ended)
-            bool occluded = spill ? trace_any_in<COUNT>(S, sr, 0.0f, ne.tmax, lds, spill, &oo, cnt)
-                                  : trace_any<COUNT>(S, sr, 0.0f, ne.tmax, lds, &oo, cnt);
-            *ovf = *ovf || oo;
-            ps.L = ps.L + (occluded ? ne.occl : ne.unoccl);
-        } else {
-            ps.L = ps.L + ne.occl;
-        }
-    }
-    // a training record's radiance so far includes the vertex's estimate
-    if (CACHE && cv.trec >= 0) cb->t_lbefore[cv.trec] = make_float4(ps.L.x, ps.L.y, ps.L.z, 0.0f);
     return more;
 }
 
-// Li from a path state to the end of the path, in one thread (the megakernel
-// from depth 0).  ps.L holds the radiance on return.
-KD v3 li_loop(const SceneView& S, const FrameConst& fc, PathState& ps, uint32_t& seed, const StackShape& lds, bool* ovf,
-              VisOut* vs) {
-    while (!is_zero(ps.beta)) {
-        if (!li_bounce(S, fc, ps, seed, lds, ovf, vs)) break;
-    }
-    return ps.L;
+// The traced estimate's term.
+template <bool CACHE = false>
+KD void li_resolve(PathState& ps, const NeeResult& ne, bool occluded, const CacheBuffers* cb = nullptr) {
+    ps.L = ps.L + (occluded ? ne.occl : ne.unoccl);
+    if (CACHE && ne.trec >= 0) cb->t_lbefore[ne.trec] = make_float4(ps.L.x, ps.L.y, ps.L.z, 0.0f);
 }
 
-// Megakernel form of Li: the whole path in one thread.
-KD v3 li_path(const SceneView& S, const FrameConst& fc, Ray ray, uint32_t& seed, const StackShape& lds, bool* ovf,
-              VisOut* vs) {
+// Megakernel form of Li: the whole path in one thread, the wave's lanes
+// vertex by vertex together (all of them call; live: the lane has a path).
+__device__ __forceinline__ v3 li_path(const SceneView& S, const FrameConst& fc, bool live, Ray ray, uint32_t& seed,
+                                      const StackShape& lds, bool* ovf, VisOut* vs) {
     PathState ps;
     ps.ray = ray;
     ps.L = mk3(0.0f, 0.0f, 0.0f);
@@ -376,7 +339,31 @@ KD v3 li_path(const SceneView& S, const FrameConst& fc, Ray ray, uint32_t& seed,
     ps.depth = 0;
     ps.p_b = 1.0f;
     ps.prev_pos = mk3(0.0f, 0.0f, 0.0f);
-    return li_loop(S, fc, ps, seed, lds, ovf, vs);
+    uint32_t spill[SPILL_STACK];
+    while (__builtin_amdgcn_ballot_w64(live) != 0ull) {
+        ClosestTrav tr;
+        tr.idle();
+        if (live) {
+            seed = seed + (uint32_t)ps.depth;
+            tr.init(S, ps.ray, 0.0f, __builtin_inff(), lds, spill);
+        }
+        tr.template run<false>(S, nullptr);
+        NeeResult ne;
+        ne.trace = false;
+        AnyTrav sh;
+        sh.idle();
+        if (live) {
+            *ovf = *ovf || tr.st.overflow();
+            live = li_shade(S, fc, ps, seed, tr.hit(), vs, &ne) && !is_zero(ps.beta);
+            if (ne.trace) sh.init(S, make_ray(ne.org, ne.dir), 0.0f, ne.tmax, lds, spill);
+        }
+        sh.template run<false>(S, nullptr);
+        if (ne.trace) {
+            *ovf = *ovf || sh.st.overflow();
+            li_resolve(ps, ne, sh.any());
+        }
+    }
+    return ps.L;
 }
 
 }  // namespace kpt

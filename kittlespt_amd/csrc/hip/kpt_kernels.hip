@@ -7,19 +7,27 @@
 namespace kpt {
 
 // ------------------------------------------------------------------ traversal
+// 8 waves per SIMD (64 VGPRs): 1125 us a million incoherent rays, 1181 at 7,
+// 1179 unconstrained (69 VGPRs).
 template <bool COUNT>
-__global__ __launch_bounds__(TRACE_BLOCK) void k_trace_closest(SceneView S, const kpt_ray* __restrict__ rays,
+__global__ __launch_bounds__(TRACE_BLOCK) __attribute__((amdgpu_waves_per_eu(8))) void k_trace_closest(SceneView S, const kpt_ray* __restrict__ rays,
                                                                kpt_hit* __restrict__ hits, int64_t n,
                                                                int32_t* overflow,
                                                                unsigned long long* counters) {
     __shared__ uint32_t s_stack[LDS_STACK][TRACE_BLOCK];
     const int64_t i = (int64_t)blockIdx.x * TRACE_BLOCK + threadIdx.x;
     TraceCounts c = {0, 0, 0, 0, 0};
+    uint32_t spill[SPILL_STACK];
+    ClosestTrav tr;
+    tr.idle();
     if (i < n) {
         const kpt_ray r = rays[i];
-        Ray w = make_ray(mk3(r.org[0], r.org[1], r.org[2]), mk3(r.dir[0], r.dir[1], r.dir[2]));
-        bool ovf = false;
-        Hit h = trace_closest<COUNT>(S, w, r.tmin, r.tmax, StackShape{&s_stack[0][threadIdx.x], TRACE_BLOCK, LDS_STACK}, &ovf, &c);
+        tr.init(S, make_ray(mk3(r.org[0], r.org[1], r.org[2]), mk3(r.dir[0], r.dir[1], r.dir[2])), r.tmin, r.tmax,
+                StackShape{&s_stack[0][threadIdx.x], TRACE_BLOCK, LDS_STACK}, spill);
+    }
+    tr.template run<COUNT>(S, &c);   // all lanes: the triangles of a leaf spread over the wave
+    if (i < n) {
+        const Hit h = tr.hit();
         kpt_hit o;
         o.t = h.t;
         if (h.slot >= 0) {
@@ -32,7 +40,7 @@ __global__ __launch_bounds__(TRACE_BLOCK) void k_trace_closest(SceneView S, cons
             o.prim_id = -1; o.inst_id = -1; o.bary[0] = 0.0f; o.bary[1] = 0.0f; o.bary[2] = 0.0f;
         }
         hits[i] = o;
-        if (ovf) atomicOr(overflow, 1);
+        if (tr.st.overflow()) atomicOr(overflow, 1);
     }
     if (COUNT) {
         // wave-level reduction, then one atomic per wave and counter
@@ -50,13 +58,19 @@ __global__ __launch_bounds__(TRACE_BLOCK) void k_trace_any(SceneView S, const kp
                                                            int32_t* overflow) {
     __shared__ uint32_t s_stack[LDS_STACK][TRACE_BLOCK];
     const int64_t i = (int64_t)blockIdx.x * TRACE_BLOCK + threadIdx.x;
-    if (i >= n) return;
-    const kpt_ray r = rays[i];
-    Ray w = make_ray(mk3(r.org[0], r.org[1], r.org[2]), mk3(r.dir[0], r.dir[1], r.dir[2]));
-    bool ovf = false;
-    bool o = trace_any<false>(S, w, r.tmin, r.tmax, StackShape{&s_stack[0][threadIdx.x], TRACE_BLOCK, LDS_STACK}, &ovf, nullptr);
-    occluded[i] = o ? 1 : 0;
-    if (ovf) atomicOr(overflow, 1);
+    uint32_t spill[SPILL_STACK];
+    AnyTrav tr;
+    tr.idle();
+    if (i < n) {
+        const kpt_ray r = rays[i];
+        tr.init(S, make_ray(mk3(r.org[0], r.org[1], r.org[2]), mk3(r.dir[0], r.dir[1], r.dir[2])), r.tmin, r.tmax,
+                StackShape{&s_stack[0][threadIdx.x], TRACE_BLOCK, LDS_STACK}, spill);
+    }
+    tr.template run<false>(S, nullptr);
+    if (i < n) {
+        occluded[i] = tr.any() ? 1 : 0;
+        if (tr.st.overflow()) atomicOr(overflow, 1);
+    }
 }
 
 hipError_t launch_trace_closest(hipStream_t s, const SceneView& S, const kpt_ray* rays, kpt_hit* hits, int64_t n,
@@ -85,10 +99,12 @@ hipError_t launch_trace_any(hipStream_t s, const SceneView& S, const kpt_ray* ra
 // computePathTraceSamplesMegaKernel (kernels.cu:385-451) with static
 // accumulation (Integrator::addSample, integrator.cuh:406-416) or temporal
 // reprojection (reprojectAccumulate, kernels.cu:299-338).  16x16 pixel
-// tiles, XCD-swizzled tile order.
+// tiles, XCD-swizzled tile order.  4 waves per SIMD (128 VGPRs): a 640x360
+// frame of depth 3 takes 1066 us, 1157 at 3 waves, 1273 unconstrained (207
+// VGPRs), 1159 at 5.
 constexpr int TILE = 16;
 
-__global__ __launch_bounds__(TRACE_BLOCK) void k_megakernel(SceneView S, FrameConst fc, int32_t frame,
+__global__ __launch_bounds__(TRACE_BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void k_megakernel(SceneView S, FrameConst fc, int32_t frame,
                                                             FrameBuffers fb, int32_t* overflow) {
     __shared__ uint32_t s_stack[LDS_STACK][TRACE_BLOCK];
     const uint32_t tiles_x = (fc.width + TILE - 1) / TILE;
@@ -96,7 +112,7 @@ __global__ __launch_bounds__(TRACE_BLOCK) void k_megakernel(SceneView S, FrameCo
     const uint32_t tile = xcd_swizzle(blockIdx.x, tiles_x * tiles_y);
     const int px = (int)((tile % tiles_x) * TILE + (threadIdx.x % TILE));
     const int py = (int)((tile / tiles_x) * TILE + (threadIdx.x / TILE));
-    if (px >= fc.width || py >= fc.height) return;
+    const bool inside = px < fc.width && py < fc.height;
     const int64_t idx = (int64_t)py * fc.width + px;
     uint32_t seed = init_seed(px, py, fc.width, frame, fc.seed_mode);
     // BoxFilter::sample consumes two numbers whose jitter is discarded (kernels.cu:397-402)
@@ -107,7 +123,8 @@ __global__ __launch_bounds__(TRACE_BLOCK) void k_megakernel(SceneView S, FrameCo
     vs.albedo = mk3(0.0f, 0.0f, 0.0f); vs.normal = mk3(0.0f, 0.0f, 0.0f); vs.pos = mk3(0.0f, 0.0f, 0.0f);
     vs.depth = __builtin_inff(); vs.inst = -1; vs.prim = -1;
     bool ovf = false;
-    v3 L = li_path(S, fc, ray, seed, StackShape{&s_stack[0][threadIdx.x], TRACE_BLOCK, LDS_STACK}, &ovf, &vs);
+    v3 L = li_path(S, fc, inside, ray, seed, StackShape{&s_stack[0][threadIdx.x], TRACE_BLOCK, LDS_STACK}, &ovf, &vs);
+    if (!inside) return;
     L = (mk3(1.0f, 1.0f, 1.0f) * 1.0f) * L;
     L = clamp_output(L);
     write_pixel(S, fc, fb, frame, idx, px, py, L, vs.albedo, vs.normal, vs.depth, vs.inst, vs.prim, vs.pos);

@@ -111,15 +111,15 @@ int bloom_levels(int width, int height);
 // TLAS rebuild on the device (kpt_tlas.hip): the host builder's tree for
 // n <= TLAS_DEVICE_MAX instance boxes (6 floats each, finite, |v| <= 1e18), in
 // the reference numbering (ref_nodes, 2n entries), the pair layout
-// (pair_nodes, 2n) and the node blocks (n + 1).  status[0] = nodes built.
+// (pair_nodes, 2n) and the traversal's pairs (n + 1).  status[0] = nodes built.
 constexpr int TLAS_DEVICE_MAX = 2048;
 hipError_t launch_tlas_build(hipStream_t s, const float* bounds, int32_t n, Node* ref_nodes, Node* pair_nodes,
-                             NodeBlock* blocks, int32_t* status);
+                             NodePair* pairs, int32_t* status);
 // TLAS refit on the device: the topology of ref_nodes (the last build, whose
 // parent[] maps every node to its parent, 0 for the root), boxes recomputed
-// from the instance boxes; then the pair layout and blocks as above.
+// from the instance boxes; then the pair layout and pairs as above.
 hipError_t launch_tlas_refit(hipStream_t s, const float* bounds, int32_t n, Node* ref_nodes, const int32_t* parent,
-                             int32_t* arrivals, Node* pair_nodes, NodeBlock* blocks, int32_t* status);
+                             int32_t* arrivals, Node* pair_nodes, NodePair* pairs, int32_t* status);
 
 // Box keys hold the slot position 3*slot+vertex+1 in 32 bits and node ids
 // are int32 (up to 2T+M): 2^29 triangles keeps both in range (and the

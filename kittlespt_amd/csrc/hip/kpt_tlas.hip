@@ -12,14 +12,15 @@
 // node.  The walk's ~2.5 N dependent scans make it slower than the host
 // builder on 1,000 instances (about 4 ms against about 1.5 ms per rebuild,
 // with 64, 128 or 256 threads), so the host builds by default; this path
-// keeps the rebuild on the stream for callers that must not wait on it.  k_tlas_layout and k_tlas_blocks then derive the traversal's pair
-// layout and two-level node blocks from it, as the host does.
+// keeps the rebuild on the stream for callers that must not wait on it.  k_tlas_layout and k_tlas_pairs then derive the traversal's pair
+// layout and the node pairs from it, as the host does.
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
 
 #include "../common/kpt_device_types.h"
 #include "kpt_launch.h"
+#include "kpt_trace.h"
 
 namespace kpt {
 namespace {
@@ -163,7 +164,7 @@ __device__ __forceinline__ Node relink(Node n, int N, uint32_t self) {
 }
 
 // Nothing is written unless the build completed (status[0] == 2N): the
-// previous layout and blocks then stay in place.
+// previous layout and pairs then stay in place.
 __global__ void k_tlas_layout(const Node* ref, int N, Node* out, const int32_t* status) {
     const int t = (int)(blockIdx.x * blockDim.x + threadIdx.x);
     if (status[0] != 2 * N) return;
@@ -184,36 +185,24 @@ __global__ void k_tlas_layout(const Node* ref, int N, Node* out, const int32_t* 
     out[2 * q + 1] = relink(ref[nb], N, nb);
 }
 
-// NodeBlock q: nodes 2q, 2q + 1 and the children of each interior one; block
-// 0 and block N stay empty, as the host's make_blocks leaves them.
-__global__ void k_tlas_blocks(const Node* pl, int N, NodeBlock* blocks, const int32_t* status) {
+// NodePair q: nodes 2q and 2q + 1 with their entries; pair 0 and pair N stay
+// empty, as the host leaves them.
+__global__ void k_tlas_pairs(const Node* pl, int N, NodePair* pairs, const int32_t* status) {
     const int q = (int)(blockIdx.x * blockDim.x + threadIdx.x);
     if (q > N || status[0] != 2 * N) return;
-    NodeBlock b{};
-    if (q >= 1 && q < N) {
-        b.c[0] = pl[2 * q];
-        b.c[1] = pl[2 * q + 1];
-        for (int k = 0; k < 2; ++k) {
-            const Node& ch = b.c[k];
-            if (ch.a != 0u && ch.a + 1u < (uint32_t)(2 * N)) {
-                b.g[2 * k] = pl[ch.a];
-                b.g[2 * k + 1] = pl[ch.a + 1];
-            }
-        }
-    }
-    blocks[q] = b;
+    pairs[q] = (q >= 1 && q < N) ? tlas_pair(pl[2 * q], pl[2 * q + 1]) : NodePair{};
 }
 
 }  // namespace
 
 hipError_t launch_tlas_build(hipStream_t s, const float* bounds, int32_t n, Node* ref_nodes, Node* pair_nodes,
-                             NodeBlock* blocks, int32_t* status) {
+                             NodePair* pairs, int32_t* status) {
     if (n <= 0 || n > TLAS_DEVICE_MAX) return hipErrorInvalidValue;
     hipLaunchKernelGGL(k_tlas_build, dim3(1), dim3(TB_THREADS), 0, s, bounds, (int)n, ref_nodes, status);
     const unsigned g1 = (unsigned)((n + 255) / 256);
     hipLaunchKernelGGL(k_tlas_layout, dim3(g1), dim3(256), 0, s, ref_nodes, (int)n, pair_nodes, status);
     const unsigned g2 = (unsigned)((n + 1 + 255) / 256);
-    hipLaunchKernelGGL(k_tlas_blocks, dim3(g2), dim3(256), 0, s, pair_nodes, (int)n, blocks, status);
+    hipLaunchKernelGGL(k_tlas_pairs, dim3(g2), dim3(256), 0, s, pair_nodes, (int)n, pairs, status);
     return hipGetLastError();
 }
 
@@ -271,7 +260,7 @@ __global__ void k_tlas_refit(const float* bounds, int N, Node* nodes, const int3
 }  // namespace
 
 hipError_t launch_tlas_refit(hipStream_t s, const float* bounds, int32_t n, Node* ref_nodes, const int32_t* parent,
-                             int32_t* arrivals, Node* pair_nodes, NodeBlock* blocks, int32_t* status) {
+                             int32_t* arrivals, Node* pair_nodes, NodePair* pairs, int32_t* status) {
     if (n <= 0) return hipErrorInvalidValue;
     const unsigned g = (unsigned)((2 * n + 255) / 256);
     hipLaunchKernelGGL(k_tlas_fill, dim3(g), dim3(256), 0, s, arrivals, 2 * n);
@@ -280,7 +269,7 @@ hipError_t launch_tlas_refit(hipStream_t s, const float* bounds, int32_t n, Node
     const unsigned g1 = (unsigned)((n + 255) / 256);
     hipLaunchKernelGGL(k_tlas_layout, dim3(g1), dim3(256), 0, s, ref_nodes, (int)n, pair_nodes, status);
     const unsigned g2 = (unsigned)((n + 1 + 255) / 256);
-    hipLaunchKernelGGL(k_tlas_blocks, dim3(g2), dim3(256), 0, s, pair_nodes, (int)n, blocks, status);
+    hipLaunchKernelGGL(k_tlas_pairs, dim3(g2), dim3(256), 0, s, pair_nodes, (int)n, pairs, status);
     return hipGetLastError();
 }
 

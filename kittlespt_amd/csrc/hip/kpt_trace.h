@@ -30,11 +30,27 @@
 //   * any-hit needs no ordering: its result is "some reachable triangle is
 //     hit", which does not depend on the visiting order; it visits the
 //     nearer child first, which finds occluders close to the origin sooner;
-//   * a node reached from its parent reuses the header words read in the
-//     parent's child test, and a leaf's triangles are loaded TRI_BATCH at a
-//     time (tested in slot order, so the closest-hit tie rule is unchanged).
-// Traversal is a state machine (init / step) so persistent kernels can refill
-// a lane with a new ray as soon as its ray finishes.
+//   * a node is represented by a 32-bit entry (below) kept in its parent's
+//     NodePair, so an interior step is one 64-byte line and nothing is decoded.
+//
+// What bounds it and what that decided (1000 instances, 1.24 M triangles,
+// 1920x1080 camera rays and their bounces).  The kernels issue vector
+// instructions for about three quarters of their cycles, and with 18 (camera
+// rays) or 9 (paths) of 64 lanes at work each, because a wave's lanes hold
+// different kinds of steps; the rest is waiting for the next node.  So a wave
+// runs one kind of step at a time (Trav::round), and the triangles of its
+// leaves are spread over all its lanes (Trav::leaves), half of a ray's work
+// and the half whose lanes were fewest.  Waiting for more lanes to reach the
+// chosen kind costs more than it fills: passes at 8, 4, 2 and 1 lanes at
+// leaves and instances took 1458, 1260, 1204 and 1125 us for a million
+// incoherent rays.  Interior steps come four to a round (a round of one:
+// 1590 us against 1458 for two, 1173 for four at two lanes).  Node pairs
+// instead of two-level 192-byte records: a third of the footprint and of the
+// cache accesses, and 64 registers instead of 96 (8 waves per SIMD instead of
+// 5).  Closest-hit launch 2.40 -> 1.51 ms, a million incoherent rays
+// 2.08 -> 1.10 ms, fifty thousand any-hit rays 124 -> 70 us.
+// Traversal is a state machine (init / round) so persistent kernels can refill
+// a lane with a new ray, and park a lane's, between rounds.
 #pragma once
 #include "kpt_vec.h"
 #include "../common/kpt_device_types.h"
@@ -43,20 +59,16 @@ namespace kpt {
 
 constexpr int TRACE_BLOCK = 256;      // threads per workgroup of the fixed-shape trace kernels
 constexpr int LDS_STACK = 16;         // stack entries per lane held in LDS (fixed-shape kernels)
-constexpr int STACK_TOTAL = 128;      // entries per lane, LDS and private together; a push beyond overflows
+constexpr int STACK_TOTAL = 128;      // entries per lane, LDS and private together (and one that marks the end);
+                                      // a push beyond overflows
 // The wavefront's persistent kernels take their LDS depth and workgroup size
 // from the tuning knobs (dynamic LDS of depth x workgroup words); the private
 // spill array is sized for the shallowest LDS part, so the total capacity is
 // STACK_TOTAL whatever the depth.
 constexpr int LDS_STACK_MIN = 8;
 constexpr int LDS_STACK_MAX = 32;
-constexpr int SPILL_STACK = STACK_TOTAL - LDS_STACK_MIN;
+constexpr int SPILL_STACK = STACK_TOTAL + 1 - LDS_STACK_MIN;
 constexpr uint32_t TLAS_BIT = 0x80000000u;
-#ifndef KPT_TRI_BATCH
-#define KPT_TRI_BATCH 4
-#endif
-constexpr int TRI_BATCH = KPT_TRI_BATCH;   // leaf triangles loaded together
-
 struct Ray {
     v3 o, d, inv;
 };
@@ -85,6 +97,14 @@ KD bool slab(const float4& lo, const float4& hi, const Ray& r, float tmin, float
     return (te <= tx) && (tx >= tmin) && (te <= tmax);
 }
 
+// The slab's entry and exit distances alone (slab above, without its tests).
+KD void slab_range(const float4& lo, const float4& hi, const Ray& r, float* tenter, float* texit) {
+    float t0x = (lo.x - r.o.x) * r.inv.x, t0y = (lo.y - r.o.y) * r.inv.y, t0z = (lo.z - r.o.z) * r.inv.z;
+    float t1x = (hi.x - r.o.x) * r.inv.x, t1y = (hi.y - r.o.y) * r.inv.y, t1z = (hi.z - r.o.z) * r.inv.z;
+    *tenter = fmaxf_(fmaxf_(fminf_(t0x, t1x), fminf_(t0y, t1y)), fminf_(t0z, t1z));
+    *texit = fminf_(fminf_(fmaxf_(t0x, t1x), fmaxf_(t0y, t1y)), fmaxf_(t0z, t1z));
+}
+
 KD void load_node(const Node* nodes, uint32_t i, float4* lo, float4* hi) {
     const float4* p = reinterpret_cast<const float4*>(nodes + i);
     *lo = p[0];
@@ -102,449 +122,375 @@ KD Ray object_ray(const InstTrav& it, const Ray& w) {
     return make_ray(o, d);
 }
 
-// Triangle::intersect (triangle.cuh:66-102) on a slot's precomputed edges.
-KD bool tri_test(const TriPos& tp, const Ray& r, float tmin, float tmax, float* t_out, float* u_out, float* v_out) {
+// Triangle::intersect (triangle.cuh:66-102) on a slot's precomputed edges
+// (a = v0, b = v1 - v0, c = v2 - v0).  The reference divides by the
+// determinant first and tests u, v and t on the quotients; here the hardware
+// reciprocal (1 ulp) rejects what lies outside by more than its error, and
+// only a triangle that may pass pays for the IEEE division and the reference's
+// own tests.  A NaN passes every one of these comparisons on to the exact
+// tests, and u > 1 is left to u + v > 1 (v is not below -1e-30).
+__device__ __forceinline__ bool triangle(const float4& a, const float4& b, const float4& c, v3 o, v3 d, float tmin,
+                                         float tmax, float* t_out, float* u_out, float* v_out) {
     const float EPS = 1.0e-5f;
-    v3 v0 = mk3(tp.v0[0], tp.v0[1], tp.v0[2]);
-    v3 e1 = mk3(tp.e1[0], tp.e1[1], tp.e1[2]);
-    v3 e2 = mk3(tp.e2[0], tp.e2[1], tp.e2[2]);
-    v3 pvec = cross(r.d, e2);
-    float det = dot(e1, pvec);
-    if (det > -EPS && det < EPS) return false;
-    float inv = 1.0f / det;
-    v3 tvec = r.o - v0;
-    float u = inv * dot(tvec, pvec);
-    if (u < 0.0f || u > 1.0f) return false;
-    v3 q = cross(tvec, e1);
-    float v = inv * dot(r.d, q);
-    if (v < 0.0f || u + v > 1.0f) return false;
-    float t = inv * dot(e2, q);
-    if (t > EPS && t < tmax && t > tmin) {
+    const v3 e1 = mk3(b.x, b.y, b.z), e2 = mk3(c.x, c.y, c.z);
+    const v3 pvec = cross(d, e2);
+    const float det = dot(e1, pvec);
+    const v3 tvec = o - mk3(a.x, a.y, a.z);
+    const float un = dot(tvec, pvec);
+    const v3 q = cross(tvec, e1);
+    const float vn = dot(d, q);
+    const float tn = dot(e2, q);
+    const float r = __builtin_amdgcn_rcpf(det);
+    const float ua = r * un, va = r * vn, ta = r * tn;
+    const float OUT = 1.00001f, NEG = -1.0e-30f;
+    bool hit = false;
+    if (!(__builtin_fabsf(det) < EPS || fminf_(fminf_(ua, va), ta) < NEG || ua + va > OUT || ta > tmax * OUT)) {
+        const float inv = 1.0f / det;
+        const float u = inv * un;
+        const float v = inv * vn;
+        const float t = inv * tn;
+        hit = !(u < 0.0f || u > 1.0f || v < 0.0f || u + v > 1.0f) && t > EPS && t < tmax && t > tmin;
         *t_out = t; *u_out = u; *v_out = v;
-        return true;
     }
-    return false;
+    return hit;
 }
 
-// Per-lane stack: LDS part [depth][stride] (stride = the workgroup's lanes,
-// so the lanes of a wave hit distinct banks) + a private spill array owned by
-// the caller (kept outside the traversal state so the state itself stays in
-// registers).
-typedef __attribute__((address_space(3))) uint32_t lds_u32;   // a pointer that is known to be LDS
+// Lane k's value (k uniform), in every lane.
+__device__ __forceinline__ float lane_of(float x, int k) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, x), k));
+}
 
 // Where a lane's stack lives: its first LDS word, the word stride between
-// entries and the number of LDS entries (LDS_STACK_MIN..LDS_STACK_MAX, or
-// LDS_STACK for the fixed-shape kernels); all but the pointer are uniform.
+// entries (a power of two: the workgroup's lanes, so the lanes of a wave hit
+// distinct banks) and the number of LDS entries (LDS_STACK_MIN..LDS_STACK_MAX,
+// or LDS_STACK for the fixed-shape kernels); all but the pointer are uniform.
 struct StackShape {
     uint32_t* lds;
     int stride;
     int depth;
 };
 
+typedef __attribute__((address_space(3))) uint32_t lds_u32;   // a pointer that is known to be LDS
+
+// Per-lane stack: LDS part [depth][stride] + a private spill array owned by
+// the caller (kept outside the traversal state so the state itself stays in
+// registers).  The top is an LDS byte address moved by the stride, so a push
+// or pop is one add and one LDS access; the lanes' first words lie within one
+// stride, so one uniform address tells for all of them whether an entry is in
+// LDS.  Entry 0 is ENTRY_IDLE: a query that pops it has ended, and no pop
+// looks for an empty stack.
 struct LaneStack {
-    lds_u32* lds;       // the lane's entry 0
+    uint32_t top;       // LDS byte address of the next free entry
     uint32_t* spill;    // private array of SPILL_STACK entries
-    int stride, depth;
-    int sp;
-    bool overflow;
-    KD void push(uint32_t e) {
-        if (sp < depth) lds[sp * stride] = e;
-        else if (sp < STACK_TOTAL) spill[sp - depth] = e;
-        else { overflow = true; return; }
-        ++sp;
+    uint32_t base;      // uniform: LDS byte address of lane 0's entry 0
+    uint32_t step;      // uniform: bytes between entries
+    uint32_t limit;     // uniform: LDS byte address past the LDS part
+    int shift;          // uniform: log2(step)
+    // entries below the address (entry 0 included); the lane's own offset is less than a step
+    KD int index(uint32_t address) const { return (int)((address - base) >> shift); }
+    KD int deep(uint32_t address) const { return (int)((address - limit) >> shift); }
+    __device__ __forceinline__ static lds_u32* at_address(uint32_t a) { return (lds_u32*)(uintptr_t)a; }
+    // A push on a full stack moves the top all the same and nothing more: the
+    // caller ends the query, and the top tells of it from then on.
+    KD bool overflow() const { return index(top) > STACK_TOTAL + 1; }
+    __device__ __forceinline__ void push(uint32_t e) {
+        if (top < limit) *at_address(top) = e;
+        else if (index(top) <= STACK_TOTAL) spill[deep(top)] = e;
+        top += step;
     }
-    KD uint32_t pop() {
-        --sp;
-        return sp < depth ? lds[sp * stride] : spill[sp - depth];
+    __device__ __forceinline__ uint32_t pop() {
+        top -= step;
+        return top < limit ? *at_address(top) : spill[deep(top)];
     }
-    // entry i (< STACK_TOTAL) read or written in place (a parked trace's copy)
-    KD uint32_t at(int i) const { return i < depth ? lds[i * stride] : spill[i - depth]; }
-    KD void set(int i, uint32_t e) {
-        if (i < depth) lds[i * stride] = e;
-        else spill[i - depth] = e;
+    // the entries above entry 0: their number, and the i-th one read or
+    // written in place (a parked trace's copy)
+    KD int size() const { return index(top) - 1; }
+    KD uint32_t address(int i) const { return top + ((uint32_t)(i - size()) << shift); }
+    __device__ __forceinline__ uint32_t get(int i) const {
+        const uint32_t a = address(i);
+        return a < limit ? *at_address(a) : spill[deep(a)];
     }
-    KD void reset(const StackShape& sh, uint32_t* spill_) {
+    __device__ __forceinline__ void reset(const StackShape& sh, uint32_t* spill_) {
         // stride and depth are the same for every lane: read them as such, so
         // they stay in scalar registers wherever the traversal runs
-        lds = (lds_u32*)sh.lds; spill = spill_;
-        stride = __builtin_amdgcn_readfirstlane(sh.stride);
-        depth = __builtin_amdgcn_readfirstlane(sh.depth);
-        sp = 0; overflow = false;
+        const uint32_t own = (uint32_t)(uintptr_t)(lds_u32*)sh.lds;
+        step = 4u * (uint32_t)__builtin_amdgcn_readfirstlane(sh.stride);
+        shift = __builtin_ctz(step);
+        base = __builtin_amdgcn_readfirstlane(own - 4u * ((uint32_t)threadIdx.x & ((step >> 2) - 1u)));
+        limit = base + (uint32_t)__builtin_amdgcn_readfirstlane(sh.depth) * step;
+        spill = spill_;
+        *at_address(own) = 0xFFFFFFFFu;
+        top = own + step;
     }
 };
 
-// ---- stack / current entries.  A BVH2 node is represented by what the
-// traversal needs to process it without loading the node itself:
-//   interior BLAS node:  pair index of its children (children at 2q, 2q+1)
-//   interior TLAS node:  TLAS_BIT | pair index of its children
-//   BLAS leaf:           LEAF_BIT | count << 23 | first slot   (count < 64, first < 2^23)
+// ---- entries.  A BVH2 node is represented by what the traversal needs to
+// process it without loading the node itself; a NodePair holds its two
+// children's boxes and entries:
+//   interior BLAS node:  index of its children's NodePair
+//   interior TLAS node:  TLAS_BIT | index of its children's NodePair
+//   BLAS leaf:           LEAF_BIT | count << 23 | first slot   (count < 64, first + count <= 2^23)
 //   larger BLAS leaf:    BIG_BIT | node index (its header is loaded)
 //   TLAS leaf:           TLAS_BIT | LEAF_BIT | instance
-// Processing an interior entry loads the 192-byte NodeBlock of its children
-// pair: both children and their children.  That replays two consecutive steps
-// of the BVH2 traversal (the node, then its nearer child when that child is
-// interior) from one block load, at the same closest distance h.t — no
-// triangle is tested between the two — so every culling decision, every push
-// and the visiting order are those of the node-at-a-time traversal.
+//   nothing left:        ENTRY_IDLE (also an empty BLAS's root entry)
+//   the stack's top:     ENTRY_POP (within a round only)
 constexpr uint32_t LEAF_BIT = 0x40000000u;
 constexpr uint32_t BIG_BIT = 0x20000000u;
 constexpr uint32_t ENTRY_PAYLOAD = 0x1FFFFFFFu;
+constexpr uint32_t ENTRY_IDLE = 0xFFFFFFFFu;
+constexpr uint32_t ENTRY_POP = 0xFFFFFFFEu;
 
 KD uint32_t bits_u(float f) { return __builtin_bit_cast(uint32_t, f); }
 
-// Entry of a BLAS child given its node index and header words.
-KD uint32_t blas_entry(uint32_t idx, uint32_t a, uint32_t b) {
-    if (b == 0u) return a >> 1;
-    if (a < (1u << 23) && b < 64u) return LEAF_BIT | (b << 23) | a;
+// Entry of a BLAS node given its index and header words; first_pair: the
+// index of the BLAS pair 0 in the pair array (the TLAS's pairs come first).
+KD uint32_t blas_entry(uint32_t idx, uint32_t a, uint32_t b, uint32_t first_pair) {
+    if (b == 0u) return first_pair + (a >> 1);
+    if (b < 64u && a + b <= (1u << 23)) return LEAF_BIT | (b << 23) | a;
     return BIG_BIT | idx;
 }
-// Entry of a TLAS child given its header words.
+// Entry of a TLAS node given its header words (pair layout).
 KD uint32_t tlas_entry(uint32_t a, uint32_t b) {
     return a != 0u ? (TLAS_BIT | (a >> 1)) : (TLAS_BIT | LEAF_BIT | b);
 }
 
-struct BlockView {
-    float4 c0l, c0h, c1l, c1h;   // children of the pair's parent
-    float4 g0l, g0h, g1l, g1h;   // children of child 0 (when interior)
-    float4 g2l, g2h, g3l, g3h;   // children of child 1 (when interior)
-};
-KD void load_block(const NodeBlock* blocks, uint32_t q, BlockView* v) {
-    const float4* p = reinterpret_cast<const float4*>(blocks + q);
-    v->c0l = p[0]; v->c0h = p[1]; v->c1l = p[2]; v->c1h = p[3];
-    v->g0l = p[4]; v->g0h = p[5]; v->g1l = p[6]; v->g1h = p[7];
-    v->g2l = p[8]; v->g2h = p[9]; v->g3l = p[10]; v->g3h = p[11];
-}
-
-// What one traversal step of a lane reads, chosen before any of it is loaded
-// so that every lane of a wave issues its loads together and the wave waits
-// for one memory round trip per step whatever mix of work its lanes hold:
-//   STEP_INTERIOR  the 192-byte NodeBlock of the entry's children pair
-//   STEP_INSTANCE  the 64-byte InstTrav of a TLAS leaf
-//   STEP_TRIS      up to TRI_BATCH 48-byte TriPos of the current leaf
-//   STEP_HEADER    the 32-byte node of a leaf too large for an entry
-enum : int { STEP_INTERIOR = 0, STEP_INSTANCE = 1, STEP_TRIS = 2, STEP_HEADER = 3 };
-constexpr int STEP_LOADS = 12;   // float4 loads per step (192 bytes)
-static_assert(3 * TRI_BATCH <= STEP_LOADS, "a triangle batch fits one step's loads");
-
-// Loads float4 [0, n) of base into v (n >= 1); the slots past n repeat the
-// last one, so the loads are issued unconditionally and stay in bounds.
-KD void step_load(const float4* base, int n, float4 v[STEP_LOADS]) {
-#pragma unroll
-    for (int k = 0; k < STEP_LOADS; ++k) v[k] = base[k < n ? k : n - 1];
-}
-
-// Classifies the lane's next step and points base/n at what it reads.  A
-// LEAF entry is decoded here (first slot and count, no load), so its first
-// triangles are read in the same step.
-KD int step_kind(const SceneView& S, uint32_t cur, uint32_t& la, uint32_t& lb, const float4** base, int* n) {
-    if (lb == 0u) {
-        if (!(cur & (LEAF_BIT | BIG_BIT))) {
-            const NodeBlock* blocks = (cur & TLAS_BIT) ? S.tlas_blocks : S.blas_blocks;
-            *base = reinterpret_cast<const float4*>(blocks + (cur & ENTRY_PAYLOAD));
-            *n = 12;
-            return STEP_INTERIOR;
-        }
-        if (cur & TLAS_BIT) {
-            *base = reinterpret_cast<const float4*>(S.inst_trav + (cur & ENTRY_PAYLOAD));
-            *n = 4;
-            return STEP_INSTANCE;
-        }
-        if (!(cur & LEAF_BIT)) {
-            *base = reinterpret_cast<const float4*>(S.blas_nodes + (cur & ENTRY_PAYLOAD));
-            *n = 2;
-            return STEP_HEADER;
-        }
-        la = cur & 0x7FFFFFu;
-        lb = (cur >> 23) & 0x3Fu;
+// The pair of two sibling nodes: tlas_pair of the TLAS's pair layout,
+// blas_pair of BLAS nodes 2q and 2q + 1.
+KD NodePair node_pair(const Node& n0, uint32_t e0, const Node& n1, uint32_t e1) {
+    NodePair p;
+    for (int k = 0; k < 3; ++k) {
+        p.lo0[k] = n0.lo[k]; p.hi0[k] = n0.hi[k];
+        p.lo1[k] = n1.lo[k]; p.hi1[k] = n1.hi[k];
     }
-    *base = reinterpret_cast<const float4*>(S.tris + la);
-    *n = 3 * (int)(lb < (uint32_t)TRI_BATCH ? lb : (uint32_t)TRI_BATCH);
-    return STEP_TRIS;
+    p.e0 = e0; p.e1 = e1; p.pad0 = 0u; p.pad1 = 0u;
+    return p;
+}
+KD NodePair tlas_pair(const Node& n0, const Node& n1) {
+    return node_pair(n0, tlas_entry(n0.a, n0.b), n1, tlas_entry(n1.a, n1.b));
+}
+KD NodePair blas_pair(const Node& n0, const Node& n1, uint32_t q, uint32_t first_pair) {
+    return node_pair(n0, blas_entry(2u * q, n0.a, n0.b, first_pair), n1,
+                     blas_entry(2u * q + 1u, n1.a, n1.b, first_pair));
 }
 
-// Closest-hit traversal state of one lane.
-struct ClosestTrav {
-    Ray w, o;
-    float tmin, tmax;
-    Hit h;
+// The least float above x (x itself for +inf and NaN): te < next_up(b) is
+// te <= b, except that te = +inf never passes.
+KD float next_up(float x) {
+    const uint32_t u = bits_u(x);
+    if (!(x < __builtin_inff())) return x;
+    return __builtin_bit_cast(float, x == 0.0f ? 1u : ((u >> 31) ? u - 1u : u + 1u));
+}
+
+constexpr int INNER_RUN = 4;   // interior steps of a round
+
+// One lane's query: ANY = false the closest hit, true any hit.
+template <bool ANY>
+struct Trav {
+    Ray w, o;           // the world ray; the current level's ray
+    float tmin;
+    float bound;        // a hit's distance has to be below this: tmax, then the closest hit so far
+    float enter;        // closest hit: a box's entry distance has to be below this
+    int32_t slot, inst; // the hit (slot -1: none)
+    float u, v;
     int32_t cur_inst;
-    uint32_t cur;
-    uint32_t la, lb;   // leaf in progress: next triangle slot, triangles left (0: none)
+    uint32_t cur;       // the entry to process next (ENTRY_IDLE: finished)
+    bool fresh;         // counting: cur is a leaf that has not been counted
     LaneStack st;
+
+    KD bool busy() const { return cur != ENTRY_IDLE; }
+    KD Hit hit() const {
+        Hit h;
+        h.t = slot >= 0 ? bound : __builtin_inff();
+        h.slot = slot; h.inst = inst; h.u = u; h.v = v;
+        return h;
+    }
+    KD bool any() const { return slot >= 0; }
+    KD void idle() { cur = ENTRY_IDLE; slot = -1; }
 
     // TLAS::intersect entry: empty TLAS or a miss of the root box ends the
-    // query at once (tlas.cu:62-69).  Returns false when nothing remains.
-    KD bool init(const SceneView& S, const Ray& ray, float t0, float t1, const StackShape& sh, uint32_t* spill) {
-        w = ray; o = ray; tmin = t0; tmax = t1;
-        h.t = __builtin_inff(); h.slot = -1; h.inst = -1; h.u = 0.0f; h.v = 0.0f;
+    // query at once (tlas.cu:62-69).
+    __device__ __forceinline__ void init(const SceneView& S, const Ray& ray, float t0, float t1, const StackShape& sh,
+                                         uint32_t* spill) {
+        w = ray; o = ray; tmin = t0; bound = t1; enter = next_up(t1);
+        slot = -1; inst = -1; u = 0.0f; v = 0.0f;
         cur_inst = -1;
-        la = 0u; lb = 0u;
+        cur = ENTRY_IDLE;
+        fresh = true;
         st.reset(sh, spill);
-        if (S.tlas_root < 0) return false;
+        if (S.tlas_root < 0) return;
         float4 rlo, rhi;
         load_node(S.tlas_nodes, 0, &rlo, &rhi);
         float te;
-        if (!slab(rlo, rhi, w, tmin, tmax, &te)) return false;
+        if (!slab(rlo, rhi, w, t0, t1, &te)) return;
         cur = tlas_entry(bits_u(rlo.w), bits_u(rhi.w));
-        return true;
     }
 
-    // Continues with the stack top; false when the stack is empty.
-    KD bool next() {
-        if (st.sp == 0 || st.overflow) return false;
-        cur = st.pop();
-        return true;
-    }
-
-    // One BVH2 interior step on the two children (l1,h1 = index i1; l2,h2 =
-    // index i2) of the node being processed: TLAS (level bit set) or BLAS.
-    // Returns 0 = nothing hit (pop), 1 = the nearer (or only) child is in
-    // *near_* (after the farther one was pushed).
-    // One code path for both levels (the level is a per-lane select), so a
-    // wave whose lanes sit at different levels does not run it twice.
-    KD bool children(bool tl, const float4& l1, const float4& h1, const float4& l2, const float4& h2, uint32_t i1,
-                     uint32_t i2, int* near_k) {
-        Ray r;
-        r.o = tl ? w.o : o.o; r.d = tl ? w.d : o.d; r.inv = tl ? w.inv : o.inv;
-        const float bt = tl ? tmax : fminf_(tmax, h.t);
-        float c1, c2;
-        const bool k1 = slab(l1, h1, r, tmin, bt, &c1) && c1 < h.t;
-        const bool k2 = slab(l2, h2, r, tmin, bt, &c2) && c2 < h.t;
-        if (k1 && k2) {
-            const bool far1 = c1 > c2;
-            const uint32_t fa = bits_u(far1 ? l1.w : l2.w), fb = bits_u(far1 ? h1.w : h2.w);
-            st.push(tl ? tlas_entry(fa, fb) : blas_entry(far1 ? i1 : i2, fa, fb));
-            *near_k = far1 ? 1 : 0;
-            return true;
+    // A lane's step leaves ENTRY_POP where the stack's top is next; an interior
+    // TLAS node is entered with the world ray again.  (The steps below are
+    // written as one-sided updates with one common pop, so that the state is
+    // updated in its registers: two-sided branches made the compiler copy it
+    // at every merge, about 40 moves a round.)
+    __device__ __forceinline__ void pop_next() {
+        bool back = false;
+        if (cur == ENTRY_POP) {
+            cur = st.pop();
+            fresh = true;
+            back = (cur & (TLAS_BIT | LEAF_BIT)) == TLAS_BIT;
         }
-        if (k1) { *near_k = 0; return true; }
-        if (k2) { *near_k = 1; return true; }
-        return false;
+        if (__builtin_amdgcn_ballot_w64(back) != 0ull) {   // uniform
+            o.o.x = back ? w.o.x : o.o.x; o.o.y = back ? w.o.y : o.o.y; o.o.z = back ? w.o.z : o.o.z;
+            o.d.x = back ? w.d.x : o.d.x; o.d.y = back ? w.d.y : o.d.y; o.d.z = back ? w.d.z : o.d.z;
+            o.inv.x = back ? w.inv.x : o.inv.x; o.inv.y = back ? w.inv.y : o.inv.y; o.inv.z = back ? w.inv.z : o.inv.z;
+        }
     }
 
-    // Processes the current entry — an interior step, an instance entry, a
-    // large leaf's header, or one batch of TRI_BATCH triangles of a leaf (a
-    // leaf spans several steps, so a wave's lanes at interior nodes are not
-    // held up by another lane's whole leaf); returns false when the query is
-    // finished.  Whatever the lane's kind of step, its reads are issued by
-    // the same instructions (step_load).
+    // Interior node: both children's boxes against the current ray; the
+    // nearer one is next, the farther one on the stack.
     template <bool COUNT>
-    KD bool step(const SceneView& S, TraceCounts* cnt) {
-        const uint32_t e = cur;
-        const bool new_leaf = (lb == 0u) && (e & LEAF_BIT) && !(e & TLAS_BIT);
-        const float4* base;
-        int n;
-        const int kind = step_kind(S, e, la, lb, &base, &n);
-        float4 v[STEP_LOADS];
-        step_load(base, n, v);
-        if (kind == STEP_INTERIOR) {
-            // interior node (TLAS or BLAS): its children pair's block
-            const bool tl = (e & TLAS_BIT) != 0;
-            const uint32_t q = e & ENTRY_PAYLOAD;
-            int nk;
-            bool any;
-            if (COUNT) { if (tl) cnt->tlas++; else cnt->interior++; }
-            any = children(tl, v[0], v[1], v[2], v[3], 2 * q, 2 * q + 1, &nk);
-            if (!any) return next();
-            if (st.overflow) return false;
-            const float4 nl = nk ? v[2] : v[0], nh = nk ? v[3] : v[1];
-            const uint32_t na = bits_u(nl.w), nb = bits_u(nh.w);
-            const bool n_interior = tl ? (na != 0u) : (nb == 0u);
-            if (!n_interior) {
-                cur = tl ? tlas_entry(na, nb) : blas_entry(2 * q + (uint32_t)nk, na, nb);
-                return true;
+    __device__ __forceinline__ void inner(const SceneView& S, TraceCounts* cnt) {
+        if (!(cur & (LEAF_BIT | BIG_BIT))) {
+            const float4* p = reinterpret_cast<const float4*>(S.pairs + (cur & ENTRY_PAYLOAD));
+            const float4 l1 = p[0], h1 = p[1], l2 = p[2], h2 = p[3];
+            if (COUNT) { if (cur & TLAS_BIT) cnt->tlas++; else cnt->interior++; }
+            float c1, c2, x1, x2;
+            slab_range(l1, h1, o, &c1, &x1);
+            slab_range(l2, h2, o, &c2, &x2);
+            const bool k1 = c1 <= x1 && x1 >= tmin && (ANY ? c1 <= bound : c1 < enter);
+            const bool k2 = c2 <= x2 && x2 >= tmin && (ANY ? c2 <= bound : c2 < enter);
+            const uint32_t e1 = bits_u(l1.w), e2 = bits_u(l2.w);
+            const bool second = k2 && (!k1 || c1 > c2);
+            cur = second ? e2 : e1;
+            cur = (k1 || k2) ? cur : ENTRY_POP;
+            fresh = true;
+            if (k1 && k2) {
+                st.push(second ? e1 : e2);
+                if (st.top > st.limit && st.overflow()) cur = ENTRY_IDLE;
             }
-            // the nearer child is interior: its step, from the same block
-            const float4 al = nk ? v[8] : v[4], ah = nk ? v[9] : v[5];
-            const float4 bl = nk ? v[10] : v[6], bh = nk ? v[11] : v[7];
-            const uint32_t p = na >> 1;   // the nearer child's children pair
-            if (COUNT) { if (tl) cnt->tlas++; else cnt->interior++; }
-            any = children(tl, al, ah, bl, bh, 2 * p, 2 * p + 1, &nk);
-            if (!any) return next();
-            if (st.overflow) return false;
-            const float4 ml = nk ? bl : al, mh = nk ? bh : ah;
-            cur = tl ? tlas_entry(bits_u(ml.w), bits_u(mh.w)) : blas_entry(2 * p + (uint32_t)nk, bits_u(ml.w), bits_u(mh.w));
-            return true;
         }
-        if (kind == STEP_INSTANCE) {
-            // TLAS leaf: enter the instance's BLAS
+        pop_next();
+    }
+
+    // TLAS leaf: the instance's BLAS, with the ray in object space.
+    template <bool COUNT>
+    __device__ __forceinline__ void instance(const SceneView& S, TraceCounts* cnt) {
+        if ((cur & (TLAS_BIT | LEAF_BIT | BIG_BIT)) == (TLAS_BIT | LEAF_BIT)) {
             if (COUNT) { cnt->tlas++; cnt->entries++; }
-            cur_inst = (int32_t)(e & ENTRY_PAYLOAD);
-            InstTrav it;
-            __builtin_memcpy(&it, v, sizeof(InstTrav));
+            cur_inst = (int32_t)(cur & ENTRY_PAYLOAD);
+            const InstTrav it = S.inst_trav[cur_inst];
             o = object_ray(it, w);
-            if (it.root_entry != 0xFFFFFFFFu) { cur = it.root_entry; return true; }
-            return next();
+            cur = it.root_entry == ENTRY_IDLE ? ENTRY_POP : it.root_entry;
+            fresh = true;
         }
-        if (kind == STEP_HEADER) {
-            // a leaf too large for an entry: its header, the triangles from the next step
-            la = bits_u(v[0].w);
-            lb = bits_u(v[1].w);
+    }
+
+    // BLAS leaves of the wave's nt lanes in ml: g = 64 / nt triangles of each,
+    // one per lane of the wave.  Lane k tests triangle k % g of the (k / g)-th
+    // of them with that lane's ray; finished lanes and lanes at other nodes
+    // work along, so the tests fill the wave however few its leaves are.  The
+    // hits are handed back one by one in lane order, which is slot order within
+    // a leaf, under the strict comparison a lane testing alone would make: the
+    // same hit, ties included.
+    template <bool COUNT>
+    __device__ __forceinline__ void leaves(const SceneView& S, TraceCounts* cnt, uint64_t ml, int nt) {
+        const int lane = (int)__lane_id();
+        const bool owner = (ml >> lane) & 1ull;
+        const int g = __builtin_amdgcn_readfirstlane((int)(64.01f * __builtin_amdgcn_rcpf((float)nt)));
+        const int inv = __builtin_amdgcn_readfirstlane((int)(4096.0f * __builtin_amdgcn_rcpf((float)g))) + 1;
+        const int r = (lane * inv) >> 12, j = lane - r * g;   // lane / g and lane % g: exact for lane < 64, g <= 64
+        // lane r of `list`: the r-th owner
+        const uint32_t below = __builtin_amdgcn_mbcnt_hi((uint32_t)(ml >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)ml, 0u));
+        const int place = owner ? (int)below : nt + lane - (int)below;
+        const int list = __builtin_amdgcn_ds_permute(4 * place, lane);
+        const int from = 4 * __builtin_amdgcn_ds_bpermute(4 * r, list);
+        auto get = [from](float x) { return __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(from, __builtin_bit_cast(int, x))); };
+        const uint32_t e = (uint32_t)__builtin_amdgcn_ds_bpermute(from, (int)cur);
+        const v3 ro = mk3(get(o.o.x), get(o.o.y), get(o.o.z)), rd = mk3(get(o.d.x), get(o.d.y), get(o.d.z));
+        const float t0 = get(tmin), t1 = get(bound);
+        const int s = (int)(e & 0x7FFFFFu) + j;
+        bool hit = false;
+        float t = 0.0f, hu = 0.0f, hv = 0.0f;
+        if (r < nt && j < (int)((e >> 23) & 0x3Fu)) {
+            const float4* p = reinterpret_cast<const float4*>(S.tris + s);
+            hit = triangle(p[0], p[1], p[2], ro, rd, t0, t1, &t, &hu, &hv);
+        }
+        const int n = (int)((cur >> 23) & 0x3Fu);
+        if (COUNT && owner) {
+            if (fresh) cnt->leaf++;
+            fresh = false;
+            cnt->tri += (uint32_t)(n < g ? n : g);
+        }
+        if (owner) cur = n > g ? cur + (uint32_t)g - ((uint32_t)g << 23) : ENTRY_POP;
+        for (uint64_t m = __builtin_amdgcn_ballot_w64(hit); m != 0ull; m &= m - 1ull) {   // uniform
+            const int k = __builtin_ctzll(m);
+            const int to = __builtin_amdgcn_readlane(from, k) >> 2;
+            const float ht = lane_of(t, k);
+            if (ANY) {
+                if (COUNT && lane == to && slot < 0) cnt->tri -= (uint32_t)((n < g ? n : g) - 1 - __builtin_amdgcn_readlane(j, k));
+                slot = lane == to ? 0 : slot;
+                cur = lane == to ? ENTRY_IDLE : cur;
+            } else {
+                const bool mine = lane == to && ht < bound;
+                slot = mine ? __builtin_amdgcn_readlane(s, k) : slot;
+                inst = mine ? cur_inst : inst;
+                u = mine ? lane_of(hu, k) : u;
+                v = mine ? lane_of(hv, k) : v;
+                bound = mine ? ht : bound;
+                enter = mine ? ht : enter;
+            }
+        }
+    }
+
+    // A leaf too large for an entry: its header, then all its triangles.
+    template <bool COUNT>
+    __device__ __forceinline__ void big_leaf(const SceneView& S, TraceCounts* cnt) {
+        if ((cur & (TLAS_BIT | LEAF_BIT | BIG_BIT)) == BIG_BIT) {
+            float4 lo, hi;
+            load_node(S.blas_nodes, cur & ENTRY_PAYLOAD, &lo, &hi);
             if (COUNT) cnt->leaf++;
-            return true;
-        }
-        if (COUNT && new_leaf) cnt->leaf++;
-        // the next TRI_BATCH triangles of the leaf, tested in slot order
-#pragma unroll
-        for (int j = 0; j < TRI_BATCH; ++j) {
-            if ((uint32_t)j < lb) {
+            const uint32_t first = bits_u(lo.w), n = bits_u(hi.w);
+            for (uint32_t j = 0; j < n && !(ANY && slot >= 0); ++j) {
+                const float4* p = reinterpret_cast<const float4*>(S.tris + first + j);
                 if (COUNT) cnt->tri++;
-                TriPos tp;
-                __builtin_memcpy(&tp, &v[3 * j], sizeof(TriPos));
-                float t, u, vv;
-                if (tri_test(tp, o, tmin, fminf_(tmax, h.t), &t, &u, &vv) && t < h.t) {
-                    h.t = t; h.slot = (int32_t)(la + j); h.inst = cur_inst; h.u = u; h.v = vv;
+                float t, hu, hv;
+                if (triangle(p[0], p[1], p[2], o.o, o.d, tmin, bound, &t, &hu, &hv)) {
+                    slot = (int32_t)(first + j); inst = cur_inst; u = hu; v = hv;
+                    if (!ANY) { bound = t; enter = t; }
                 }
             }
+            cur = (ANY && slot >= 0) ? ENTRY_IDLE : ENTRY_POP;
         }
-        if (lb > (uint32_t)TRI_BATCH) { la += TRI_BATCH; lb -= TRI_BATCH; return true; }
-        lb = 0u;
-        return next();
     }
-};
 
-// Any-hit traversal state of one lane (entries and blocks as above; no
-// closest-distance bound, nearer child first).
-struct AnyTrav {
-    Ray w, o;
-    float tmin, tmax;
-    bool hit;
-    uint32_t cur;
-    uint32_t la, lb;
-    LaneStack st;
-
-    KD bool init(const SceneView& S, const Ray& ray, float t0, float t1, const StackShape& sh, uint32_t* spill) {
-        w = ray; o = ray; tmin = t0; tmax = t1; hit = false;
-        la = 0u; lb = 0u;
-        st.reset(sh, spill);
-        if (S.tlas_root < 0) return false;
-        float4 rlo, rhi;
-        load_node(S.tlas_nodes, 0, &rlo, &rhi);
-        float te;
-        if (!slab(rlo, rhi, w, tmin, tmax, &te)) return false;
-        cur = tlas_entry(bits_u(rlo.w), bits_u(rhi.w));
-        return true;
-    }
-    KD bool next() {
-        if (st.sp == 0 || st.overflow) return false;
-        cur = st.pop();
-        return true;
-    }
-    KD bool children(bool tl, const float4& l1, const float4& h1, const float4& l2, const float4& h2, uint32_t i1,
-                     uint32_t i2, int* near_k) {
-        Ray r;
-        r.o = tl ? w.o : o.o; r.d = tl ? w.d : o.d; r.inv = tl ? w.inv : o.inv;
-        float c1, c2;
-        const bool k1 = slab(l1, h1, r, tmin, tmax, &c1);
-        const bool k2 = slab(l2, h2, r, tmin, tmax, &c2);
-        if (k1 && k2) {   // nearer first: an occluder near the origin ends the query sooner
-            const bool far1 = c1 > c2;
-            const uint32_t fa = bits_u(far1 ? l1.w : l2.w), fb = bits_u(far1 ? h1.w : h2.w);
-            st.push(tl ? tlas_entry(fa, fb) : blas_entry(far1 ? i1 : i2, fa, fb));
-            *near_k = far1 ? 1 : 0;
-            return true;
-        }
-        if (k1) { *near_k = 0; return true; }
-        if (k2) { *near_k = 1; return true; }
-        return false;
-    }
+    // One round of the wave, called with all its lanes active (finished ones
+    // help with the triangles): a pass over its leaves, one over its instances,
+    // then INNER_RUN interior steps.
     template <bool COUNT>
-    KD bool step(const SceneView& S, TraceCounts* cnt) {
-        const uint32_t e = cur;
-        const bool new_leaf = (lb == 0u) && (e & LEAF_BIT) && !(e & TLAS_BIT);
-        const float4* base;
-        int n;
-        const int kind = step_kind(S, e, la, lb, &base, &n);
-        float4 v[STEP_LOADS];
-        step_load(base, n, v);
-        if (kind == STEP_INTERIOR) {
-            const bool tl = (e & TLAS_BIT) != 0;
-            const uint32_t q = e & ENTRY_PAYLOAD;
-            int nk;
-            bool any;
-            if (COUNT) { if (tl) cnt->tlas++; else cnt->interior++; }
-            any = children(tl, v[0], v[1], v[2], v[3], 2 * q, 2 * q + 1, &nk);
-            if (!any) return next();
-            if (st.overflow) return false;
-            const float4 nl = nk ? v[2] : v[0], nh = nk ? v[3] : v[1];
-            const uint32_t na = bits_u(nl.w), nb = bits_u(nh.w);
-            const bool n_interior = tl ? (na != 0u) : (nb == 0u);
-            if (!n_interior) {
-                cur = tl ? tlas_entry(na, nb) : blas_entry(2 * q + (uint32_t)nk, na, nb);
-                return true;
-            }
-            const float4 al = nk ? v[8] : v[4], ah = nk ? v[9] : v[5];
-            const float4 bl = nk ? v[10] : v[6], bh = nk ? v[11] : v[7];
-            const uint32_t p = na >> 1;
-            if (COUNT) { if (tl) cnt->tlas++; else cnt->interior++; }
-            any = children(tl, al, ah, bl, bh, 2 * p, 2 * p + 1, &nk);
-            if (!any) return next();
-            if (st.overflow) return false;
-            const float4 ml = nk ? bl : al, mh = nk ? bh : ah;
-            cur = tl ? tlas_entry(bits_u(ml.w), bits_u(mh.w)) : blas_entry(2 * p + (uint32_t)nk, bits_u(ml.w), bits_u(mh.w));
-            return true;
-        }
-        if (kind == STEP_INSTANCE) {
-            if (COUNT) { cnt->tlas++; cnt->entries++; }
-            InstTrav it;
-            __builtin_memcpy(&it, v, sizeof(InstTrav));
-            o = object_ray(it, w);
-            if (it.root_entry != 0xFFFFFFFFu) { cur = it.root_entry; return true; }
-            return next();
-        }
-        if (kind == STEP_HEADER) {
-            la = bits_u(v[0].w);
-            lb = bits_u(v[1].w);
-            if (COUNT) cnt->leaf++;
-            return true;
-        }
-        if (COUNT && new_leaf) cnt->leaf++;
+    __device__ __forceinline__ void round(const SceneView& S, TraceCounts* cnt) {
+        const uint32_t kind = cur & (TLAS_BIT | LEAF_BIT | BIG_BIT);
+        const uint64_t ml = __builtin_amdgcn_ballot_w64(kind == LEAF_BIT);
+        if (ml != 0ull) {
+            leaves<COUNT>(S, cnt, ml, __builtin_popcountll(ml));
+            pop_next();
+        } else if (__builtin_amdgcn_ballot_w64(kind == (TLAS_BIT | LEAF_BIT)) != 0ull) {
+            instance<COUNT>(S, cnt);
+            pop_next();
+        } else if (__builtin_amdgcn_ballot_w64(!(cur & (LEAF_BIT | BIG_BIT))) != 0ull) {
 #pragma unroll
-        for (int j = 0; j < TRI_BATCH; ++j) {
-            if ((uint32_t)j < lb) {
-                if (COUNT) cnt->tri++;
-                TriPos tp;
-                __builtin_memcpy(&tp, &v[3 * j], sizeof(TriPos));
-                float t, u, vv;
-                if (tri_test(tp, o, tmin, tmax, &t, &u, &vv)) { hit = true; lb = 0u; return false; }
-            }
+            for (int k = 0; k < INNER_RUN; ++k) inner<COUNT>(S, cnt);
+        } else {
+            big_leaf<COUNT>(S, cnt);
+            pop_next();
         }
-        if (lb > (uint32_t)TRI_BATCH) { la += TRI_BATCH; lb -= TRI_BATCH; return true; }
-        lb = 0u;
-        return next();
+    }
+
+    // To the end of every lane's query (all lanes of the wave active).
+    template <bool COUNT>
+    __device__ __forceinline__ void run(const SceneView& S, TraceCounts* cnt) {
+        while (__builtin_amdgcn_ballot_w64(busy()) != 0ull) round<COUNT>(S, cnt);
     }
 };
-
-// Whole-query forms (megakernel, trace entry points, the wavefront's tail).
-template <bool COUNT>
-KD Hit trace_closest(const SceneView& S, const Ray& w, float tmin, float tmax, const StackShape& sh,
-                     bool* overflow, TraceCounts* cnt) {
-    uint32_t spill[SPILL_STACK];
-    ClosestTrav tr;
-    if (tr.init(S, w, tmin, tmax, sh, spill)) {
-        while (tr.template step<COUNT>(S, cnt)) {}
-    }
-    *overflow = tr.st.overflow;
-    return tr.h;
-}
-
-template <bool COUNT>
-KD bool trace_any_in(const SceneView& S, const Ray& w, float tmin, float tmax, const StackShape& sh, uint32_t* spill,
-                     bool* overflow, TraceCounts* cnt) {
-    AnyTrav tr;
-    if (tr.init(S, w, tmin, tmax, sh, spill)) {
-        while (tr.template step<COUNT>(S, cnt)) {}
-    }
-    *overflow = tr.st.overflow;
-    return tr.hit;
-}
-
-template <bool COUNT>
-KD bool trace_any(const SceneView& S, const Ray& w, float tmin, float tmax, const StackShape& sh, bool* overflow,
-                  TraceCounts* cnt) {
-    uint32_t spill[SPILL_STACK];
-    return trace_any_in<COUNT>(S, w, tmin, tmax, sh, spill, overflow, cnt);
-}
+typedef Trav<false> ClosestTrav;
+typedef Trav<true> AnyTrav;
 
 // XCD-aware workgroup swizzle: the dispatcher hands consecutive workgroup ids
 // to the 8 XCDs round-robin; remap so each XCD owns a contiguous run of tiles

@@ -22,19 +22,13 @@ namespace {
 
 constexpr int WF_BLOCK = 256;
 // Occupancy targets in waves per SIMD (512 VGPRs per lane per SIMD): the
-// traversal kernels at 5 (at most 96 VGPRs; they need 100 unconstrained and
-// fit without spilling), the path-per-lane tail at 4 (128 VGPRs, from 166).
-// Both measured faster than the unconstrained allocation on the instanced
-// 1080p workload.
-#ifndef KPT_WPE_TRACE
-#define KPT_WPE_TRACE __attribute__((amdgpu_waves_per_eu(5)))
-#endif
-#ifndef KPT_WPE_TAIL
-#define KPT_WPE_TAIL __attribute__((amdgpu_waves_per_eu(4)))
-#endif
-#ifndef KPT_WPE_SHADE
-#define KPT_WPE_SHADE
-#endif
+// traversal kernels at 8 (64 VGPRs; the closest-hit launch of a 1080p frame
+// 1.54 ms, 1.62 at 6 waves), the path-per-lane tail at 5 (96 VGPRs with the
+// path's state spilled around its traversals: 4.01 ms, 4.09 at 4 waves, 4.69
+// at 3, and 5.0 to 5.8 at 6).
+#define KPT_WPE_TRACE __attribute__((amdgpu_waves_per_eu(8)))
+#define KPT_WPE_TAIL __attribute__((amdgpu_waves_per_eu(5)))
+constexpr int TRACE_ROUNDS = 8;   // traversal rounds of a wave between looks at its idle lanes
 constexpr int MAX_KEYS = 64;
 // counters[] slots (zeroed once per frame by a fill kernel)
 constexpr int C_QCOUNT = 0;      // + bounce parity: [0],[1] live-queue sizes
@@ -62,35 +56,6 @@ __device__ __forceinline__ int wave_claim(int32_t* ctr, int n) {
     if (lane_id() == 0) base = atomicAdd(ctr, n);
     return __shfl(base, 0, WAVE);
 }
-
-// Wave-local work source over a global queue of `count` entries: a wave claims
-// `chunk` entries at a time and hands them to its idle lanes (once at least
-// `refill_min` are idle), so a lane whose ray finishes starts another without
-// waiting for the rest of the wave.
-struct WaveFeeder {
-    int pos, end;        // wave-uniform claimed range [pos, end)
-    bool drained;
-    int chunk, refill_min;
-    __device__ void init(const TraceTuning& t) {
-        pos = 0; end = 0; drained = false; chunk = t.chunk; refill_min = t.refill_min;
-    }
-    // Returns the queue position for this lane (when `idle`) or -1.
-    __device__ int feed(int32_t* ctr, int count, bool idle) {
-        const uint64_t m = __ballot(idle);
-        const int n = __popcll(m);
-        if (n == 0 || (n < refill_min && n < WAVE)) return -1;
-        if (pos >= end && !drained) {
-            int b = wave_claim(ctr, chunk);
-            if (b >= count) drained = true;
-            else { pos = b; end = min(b + chunk, count); }
-        }
-        if (pos >= end) return -1;
-        const int k = pos + __popcll(m & lanes_below());
-        pos = min(pos + n, end);
-        return (idle && k < end) ? k : -1;
-    }
-    __device__ bool exhausted() const { return drained && pos >= end; }
-};
 
 __global__ void k_fill_i32(int32_t* p, int32_t v, int n) {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -250,64 +215,52 @@ __global__ __launch_bounds__(WF_BLOCK) KPT_WPE_TRACE void k_trace(SceneView S, W
     const StackShape lds{s_dyn + threadIdx.x, (int)blockDim.x, tune.stack};
     bool ovf = false;
     TraceCounts c = {0, 0, 0, 0, 0};
-    if (!tune.refill) {
-        // one ray per lane to completion; a wave claims tune.chunk entries
-        // (a multiple of 64) per atomic and runs them 64 at a time
-        const int chunk = (tune.chunk / WAVE) * WAVE;
-        for (;;) {
-            const int base = wave_claim(ctr, chunk);
-            if (base >= count) break;
-            for (int off = 0; off < chunk && base + off < count; off += WAVE) {
-                const int k = base + off + lane_id();
-                if (k >= count) continue;
-                const int p = q[k];
-                const float4 o = W.ray_o[p], d = W.ray_d[p];
-                const uint32_t b0 = c.interior + c.leaf, t0 = c.tlas;
-                ClosestTrav tr;
-                if (tr.init(S, make_ray(mk3(o.x, o.y, o.z), mk3(d.x, d.y, d.z)), 0.0f, __builtin_inff(), lds,
-                            spill)) {
-                    while (tr.template step<COUNT>(S, &c)) {}
+    // A wave's lanes take queue entries 64 at a time (refill off: once all its
+    // rays have ended; on: once at least refill_min lanes are idle), from
+    // claims of tune.chunk entries (a multiple of 64) per atomic.  A lane
+    // writes its hit when the wave takes new rays, not when its own ray ends.
+    const int refill_min = tune.refill ? tune.refill_min : WAVE;
+    const int chunk = max(tune.chunk / WAVE, 1) * WAVE;
+    int pos = 0, end = 0;     // wave-uniform: the claimed range [pos, end)
+    bool drained = false;
+    ClosestTrav tr;
+    tr.idle();
+    int p = -1;               // the lane's path, until its hit is written
+    uint32_t b0 = 0u, t0 = 0u;   // counting mode: the lane's counts when its ray started
+    float pix = 0.0f;
+    for (;;) {
+        const uint64_t m = __ballot(!tr.busy());
+        const int idle = __popcll(m);
+        if (idle >= refill_min && !(drained && pos >= end && idle < WAVE)) {
+            if (!tr.busy()) {
+                if (p >= 0) {
+                    const Hit h = tr.hit();
+                    ovf = ovf || tr.st.overflow();
+                    if (COUNT && W.heat) heat_add(W.heat, pix, c.interior + c.leaf - b0, c.tlas - t0);
+                    W.hit[p] = make_float4(h.t, bitsf((uint32_t)h.slot), bitsf((uint32_t)h.inst), h.u);
+                    W.hit_v[p] = h.v;
+                    p = -1;
                 }
-                if (COUNT && W.heat) heat_add(W.heat, o.w, c.interior + c.leaf - b0, c.tlas - t0);
-                ovf = ovf || tr.st.overflow;
-                W.hit[p] = make_float4(tr.h.t, bitsf((uint32_t)tr.h.slot), bitsf((uint32_t)tr.h.inst), tr.h.u);
-                W.hit_v[p] = tr.h.v;
             }
-        }
-    } else {
-        WaveFeeder feeder;
-        feeder.init(tune);
-        ClosestTrav tr;
-        int p = -1;
-        bool busy = false;
-        uint32_t b0 = 0u, t0 = 0u;   // counting mode: the lane's counts when its ray started
-        float pix = 0.0f;
-        for (;;) {
-            const int k = feeder.feed(ctr, count, !busy);
-            bool done_now = false;
-            if (k >= 0) {
+            if (pos >= end && !drained) {
+                const int b = wave_claim(ctr, chunk);
+                if (b >= count) drained = true;
+                else { pos = b; end = min(b + chunk, count); }
+            }
+            if (pos >= end) {
+                if (idle == WAVE) break;
+                continue;
+            }
+            const int k = pos + __popcll(m & lanes_below());
+            pos = min(pos + idle, end);
+            if (!tr.busy() && k < end) {
                 p = q[k];
                 const float4 o = W.ray_o[p], d = W.ray_d[p];
                 if (COUNT) { b0 = c.interior + c.leaf; t0 = c.tlas; pix = o.w; }
-                busy = tr.init(S, make_ray(mk3(o.x, o.y, o.z), mk3(d.x, d.y, d.z)), 0.0f, __builtin_inff(), lds,
-                               spill);
-                done_now = !busy;   // empty scene or root box missed
-            }
-            if (!__any(busy || done_now)) {   // wave-uniform
-                if (feeder.exhausted()) break;
-                continue;
-            }
-            if (busy) {
-                busy = tr.template step<COUNT>(S, &c);
-                done_now = !busy;
-            }
-            if (done_now) {
-                ovf = ovf || tr.st.overflow;
-                if (COUNT && W.heat) heat_add(W.heat, pix, c.interior + c.leaf - b0, c.tlas - t0);
-                W.hit[p] = make_float4(tr.h.t, bitsf((uint32_t)tr.h.slot), bitsf((uint32_t)tr.h.inst), tr.h.u);
-                W.hit_v[p] = tr.h.v;
+                tr.init(S, make_ray(mk3(o.x, o.y, o.z), mk3(d.x, d.y, d.z)), 0.0f, __builtin_inff(), lds, spill);
             }
         }
+        for (int j = 0; j < TRACE_ROUNDS && __builtin_amdgcn_ballot_w64(tr.busy()) != 0ull; ++j) tr.template round<COUNT>(S, &c);
     }
     if (ovf) atomicOr(overflow, 1);
     if (COUNT) {
@@ -380,7 +333,7 @@ __global__ __launch_bounds__(WF_BLOCK) void k_sort_scatter(SceneView S, Wavefron
 // its waves' ballots in LDS): the appends of every workgroup target the same
 // two counters, and one atomic per 256 lanes instead of one per wave and
 // queue keeps that address's queue in L2 short.
-__global__ __launch_bounds__(WF_BLOCK) KPT_WPE_SHADE void k_shade(SceneView S, FrameConst fc, WavefrontState W, int parity,
+__global__ __launch_bounds__(WF_BLOCK) void k_shade(SceneView S, FrameConst fc, WavefrontState W, int parity,
                                                     const int32_t* q, CacheBuffers cb, CacheFrame cf) {
     constexpr int NW = WF_BLOCK / WAVE;
     __shared__ int s_off[2][NW + 1];   // per queue: the waves' offsets, then the workgroup's base
@@ -518,7 +471,7 @@ __global__ __launch_bounds__(WF_BLOCK) KPT_WPE_SHADE void k_shade(SceneView S, F
     if (alive) W.queue[parity ^ 1][s_off[1][NW] + s_off[1][wave] + __popcll(m_al & lanes_below())] = p;
 }
 
-// The rest of every path still alive, one path per lane (li_bounce from the
+// The rest of every path still alive, one path per lane (li_shade from the
 // path's state in HBM): after the first bounces few paths remain, each needing
 // several dependent trace/shade/shadow rounds, and per-bounce launches would
 // be bound by the latency of their few rays.  Same arithmetic and random
@@ -538,16 +491,16 @@ __global__ __launch_bounds__(WF_BLOCK) KPT_WPE_SHADE void k_shade(SceneView S, F
 // lane goes on as an idle lane.  Idle lanes take parked traces before new
 // paths, load the path as a claimed one and continue the traversal from the
 // state it stopped in, so every ray runs the same steps in the same order and
-// the image is unchanged.  Each parked trace has run at least one step since
-// it was begun or taken back, and a wave that has drained the queue parks
-// nothing, so every trace ends.
+// the image is unchanged.  A wave that parks traces claims new paths in their
+// place, and one that has drained the queue parks nothing, so every trace
+// ends.
 // CACHE: the radiance cache's hooks at each path's cache vertex (li_shade).
 constexpr int TAIL_POOL = 64;         // parked traces per wave
 constexpr int TAIL_SLOT_HEAD = 4;     // float4 of a parked trace's state before its stack
 constexpr int TAIL_SAVE_STACK = 48;   // stack entries a parked trace may hold
 constexpr int TAIL_SLOT_F4 = TAIL_SLOT_HEAD + TAIL_SAVE_STACK / 4;   // float4 per parked trace
 static_assert(TAIL_POOL * TAIL_SLOT_F4 * 16 == TAIL_POOL_BYTES, "pool layout");
-constexpr int TAIL_CHECK = 16;        // trace steps per lane between parking checks
+constexpr int TAIL_CHECK = 32;        // traversal rounds between parking checks
 
 template <bool COUNT, bool CACHE>
 __global__ __launch_bounds__(WF_BLOCK) KPT_WPE_TAIL void k_tail(SceneView S, FrameConst fc, WavefrontState W, int parity,
@@ -617,91 +570,102 @@ __global__ __launch_bounds__(WF_BLOCK) KPT_WPE_TAIL void k_tail(SceneView S, Fra
             if (COUNT && W.heat) heat_px = W.heat + 2 * (int64_t)fbits(o4.w);
         }
         if (!__any(active)) break;   // wave-uniform: queue drained, nothing parked, every lane idle
-        // the vertex's closest-hit trace: begun here, or taken back where it was parked
+        // the vertex's closest-hit trace: begun here, or taken back where it was
+        // parked.  All lanes go through the traversals, with or without a query
+        // of their own: the triangles of a leaf are spread over the wave.
         bool missed = false, parked = false;
-        if (active) {
-            bool o = false, more = false;
-            if (resumed || !is_zero(ps.beta)) {
-                ClosestTrav tr;
-                bool busy = true;
-                if (resumed) {
-                    // the world ray is the path's ray (as the trace was begun with it), the
-                    // object ray recomputed from it as the instance step computed it
-                    const float4* sl = pool + slot * TAIL_SLOT_F4;
-                    const float4 a0 = sl[0], a1 = sl[1], a2 = sl[2], a3 = sl[3];
-                    tr.w = ps.ray;
-                    tr.tmin = a0.y; tr.tmax = a0.z; tr.h.t = a0.w;
-                    tr.h.slot = (int32_t)fbits(a1.x); tr.h.inst = (int32_t)fbits(a1.y); tr.h.u = a1.z; tr.h.v = a1.w;
-                    tr.cur_inst = (int32_t)fbits(a2.x); tr.cur = fbits(a2.y); tr.la = fbits(a2.z); tr.lb = fbits(a2.w);
-                    const int sp = (int)fbits(a3.x);
-                    tr.o = tr.cur_inst >= 0 ? object_ray(S.inst_trav[tr.cur_inst], tr.w) : tr.w;
-                    tr.st.reset(lds, spill);
-                    for (int i = 0; i < sp; i += 4) {
-                        const float4 e = sl[TAIL_SLOT_HEAD + i / 4];
-                        tr.st.set(i, fbits(e.x));
-                        if (i + 1 < sp) tr.st.set(i + 1, fbits(e.y));
-                        if (i + 2 < sp) tr.st.set(i + 2, fbits(e.z));
-                        if (i + 3 < sp) tr.st.set(i + 3, fbits(e.w));
-                    }
-                    tr.st.sp = sp;
-                } else {
-                    if (COUNT) ++n_vertices;
-                    seed = seed + (uint32_t)ps.depth;
-                    busy = tr.init(S, ps.ray, 0.0f, __builtin_inff(), lds, spill);
+        const bool tracing = active && (resumed || !is_zero(ps.beta));
+        ClosestTrav tr;
+        tr.idle();
+        if (tracing) {
+            if (resumed) {
+                // the world ray is the path's ray (as the trace was begun with it), the
+                // object ray recomputed from it as the instance step computed it
+                const float4* sl = pool + slot * TAIL_SLOT_F4;
+                const float4 a0 = sl[0], a1 = sl[1], a2 = sl[2], a3 = sl[3];
+                tr.w = ps.ray;
+                tr.tmin = a0.y; tr.bound = a0.z; tr.enter = a0.w;
+                tr.slot = (int32_t)fbits(a1.x); tr.inst = (int32_t)fbits(a1.y); tr.u = a1.z; tr.v = a1.w;
+                tr.cur_inst = (int32_t)fbits(a2.x); tr.cur = fbits(a2.y); tr.fresh = fbits(a2.z) != 0u;
+                const int sp = (int)fbits(a3.x);
+                tr.o = (tr.cur & TLAS_BIT) ? tr.w : object_ray(S.inst_trav[tr.cur_inst], tr.w);
+                tr.st.reset(lds, spill);
+                for (int i = 0; i < sp; i += 4) {
+                    const float4 e = sl[TAIL_SLOT_HEAD + i / 4];
+                    tr.st.push(fbits(e.x));
+                    if (i + 1 < sp) tr.st.push(fbits(e.y));
+                    if (i + 2 < sp) tr.st.push(fbits(e.z));
+                    if (i + 3 < sp) tr.st.push(fbits(e.w));
                 }
-                const uint32_t b0 = COUNT ? c.interior + c.leaf : 0u, t0 = COUNT ? c.tlas : 0u;
-                // TAIL_CHECK steps per lane between looks at how many lanes still trace
-                for (;;) {
-                    for (int j = 0; j < TAIL_CHECK && busy; ++j) busy = tr.template step<COUNT>(S, &c);
-                    const uint64_t m = __ballot(busy);   // the same for every lane in here
-                    if (m == 0ull) break;
-                    if (pool && !drained && __popcll(m) < suspend && __popcll(m) <= TAIL_POOL - npool &&
-                        __ballot(busy && tr.st.sp > TAIL_SAVE_STACK) == 0ull)
-                        break;
-                }
-                if (COUNT && heat_px) {
-                    atomicAdd(&heat_px[0], (int32_t)(c.interior + c.leaf - b0));
-                    atomicAdd(&heat_px[1], (int32_t)(c.tlas - t0));
-                }
-                // the traces still running are parked in the wave's slots from npool on
-                const uint64_t mp = __ballot(busy);
-                if (busy) {
-                    // the path as a queued one (seed already advanced: its trace has begun); the
-                    // pixel in the origin's w stays
-                    *reinterpret_cast<float3*>(&W.ray_o[p]) = make_float3(ps.ray.o.x, ps.ray.o.y, ps.ray.o.z);
-                    W.ray_d[p] = make_float4(ps.ray.d.x, ps.ray.d.y, ps.ray.d.z, bitsf(seed));
-                    W.beta[p] = make_float4(ps.beta.x, ps.beta.y, ps.beta.z, ps.p_b);
-                    W.L[p] = make_float4(ps.L.x, ps.L.y, ps.L.z,
-                                         bitsf((uint32_t)ps.depth | (ps.any_nonspec ? 0x10000u : 0u) |
-                                               (ps.wide_in ? 0x20000u : 0u) | (ps.cached ? 0x40000u : 0u)));
-                    W.prev_pos[p] = make_float4(ps.prev_pos.x, ps.prev_pos.y, ps.prev_pos.z, 0.0f);
-                    float4* sl = pool + (npool + __popcll(mp & lanes_below())) * TAIL_SLOT_F4;
-                    const int sp = tr.st.sp;
-                    sl[0] = make_float4(bitsf((uint32_t)p), tr.tmin, tr.tmax, tr.h.t);
-                    sl[1] = make_float4(bitsf((uint32_t)tr.h.slot), bitsf((uint32_t)tr.h.inst), tr.h.u, tr.h.v);
-                    sl[2] = make_float4(bitsf((uint32_t)tr.cur_inst), bitsf(tr.cur), bitsf(tr.la), bitsf(tr.lb));
-                    sl[3] = make_float4(bitsf((uint32_t)sp), 0.0f, 0.0f, 0.0f);
-                    for (int i = 0; i < sp; i += 4) {
-                        const uint32_t e0 = tr.st.at(i);
-                        const uint32_t e1 = i + 1 < sp ? tr.st.at(i + 1) : 0u;
-                        const uint32_t e2 = i + 2 < sp ? tr.st.at(i + 2) : 0u;
-                        const uint32_t e3 = i + 3 < sp ? tr.st.at(i + 3) : 0u;
-                        sl[TAIL_SLOT_HEAD + i / 4] = make_float4(bitsf(e0), bitsf(e1), bitsf(e2), bitsf(e3));
-                    }
-                    parked = true;
-                } else {
-                    o = tr.st.overflow;
-                    more = li_shade<COUNT, true, CACHE>(S, fc, ps, seed, tr.h, lds, &o, &vs, &c, &missed, &cb, &cf,
-                                                        p, spill);
-                }
+            } else {
+                if (COUNT) ++n_vertices;
+                seed = seed + (uint32_t)ps.depth;
+                tr.init(S, ps.ray, 0.0f, __builtin_inff(), lds, spill);
             }
-            ovf = ovf || o;
-            if (parked) {
-                active = false;
-            } else if (!more || is_zero(ps.beta)) {
-                W.L[p] = make_float4(ps.L.x, ps.L.y, ps.L.z, bitsf((uint32_t)ps.depth | (st & 0x10000u)));
-                active = false;
+        }
+        const uint32_t b0 = COUNT ? c.interior + c.leaf : 0u, t0 = COUNT ? c.tlas : 0u;
+        // TAIL_CHECK rounds between looks at how many lanes still trace
+        uint64_t mp = 0ull;   // the traces to park
+        for (;;) {
+            for (int j = 0; j < TAIL_CHECK && __builtin_amdgcn_ballot_w64(tr.busy()) != 0ull; ++j)
+                tr.template round<COUNT>(S, &c);
+            mp = __ballot(tr.busy());
+            if (mp == 0ull) break;
+            if (pool && !drained && __popcll(mp) < suspend && __popcll(mp) <= TAIL_POOL - npool &&
+                __ballot(tr.busy() && tr.st.size() > TAIL_SAVE_STACK) == 0ull)
+                break;
+        }
+        if (COUNT && heat_px && tracing) {
+            atomicAdd(&heat_px[0], (int32_t)(c.interior + c.leaf - b0));
+            atomicAdd(&heat_px[1], (int32_t)(c.tlas - t0));
+        }
+        // the traces still running are parked in the wave's slots from npool on
+        if (tr.busy()) {
+            // the path as a queued one (seed already advanced: its trace has begun); the
+            // pixel in the origin's w stays
+            *reinterpret_cast<float3*>(&W.ray_o[p]) = make_float3(ps.ray.o.x, ps.ray.o.y, ps.ray.o.z);
+            W.ray_d[p] = make_float4(ps.ray.d.x, ps.ray.d.y, ps.ray.d.z, bitsf(seed));
+            W.beta[p] = make_float4(ps.beta.x, ps.beta.y, ps.beta.z, ps.p_b);
+            W.L[p] = make_float4(ps.L.x, ps.L.y, ps.L.z,
+                                 bitsf((uint32_t)ps.depth | (ps.any_nonspec ? 0x10000u : 0u) |
+                                       (ps.wide_in ? 0x20000u : 0u) | (ps.cached ? 0x40000u : 0u)));
+            W.prev_pos[p] = make_float4(ps.prev_pos.x, ps.prev_pos.y, ps.prev_pos.z, 0.0f);
+            float4* sl = pool + (npool + __popcll(mp & lanes_below())) * TAIL_SLOT_F4;
+            const int sp = tr.st.size();
+            sl[0] = make_float4(bitsf((uint32_t)p), tr.tmin, tr.bound, tr.enter);
+            sl[1] = make_float4(bitsf((uint32_t)tr.slot), bitsf((uint32_t)tr.inst), tr.u, tr.v);
+            sl[2] = make_float4(bitsf((uint32_t)tr.cur_inst), bitsf(tr.cur), bitsf(tr.fresh ? 1u : 0u), 0.0f);
+            sl[3] = make_float4(bitsf((uint32_t)sp), 0.0f, 0.0f, 0.0f);
+            for (int i = 0; i < sp; i += 4) {
+                const uint32_t e0 = tr.st.get(i);
+                const uint32_t e1 = i + 1 < sp ? tr.st.get(i + 1) : 0u;
+                const uint32_t e2 = i + 2 < sp ? tr.st.get(i + 2) : 0u;
+                const uint32_t e3 = i + 3 < sp ? tr.st.get(i + 3) : 0u;
+                sl[TAIL_SLOT_HEAD + i / 4] = make_float4(bitsf(e0), bitsf(e1), bitsf(e2), bitsf(e3));
             }
+            parked = true;
+        }
+        // shading, then the wave's shadow rays
+        bool more = false;
+        NeeResult ne;
+        ne.trace = false;
+        AnyTrav sh;
+        sh.idle();
+        if (tracing && !parked) {
+            ovf = ovf || tr.st.overflow();
+            more = li_shade<true, CACHE>(S, fc, ps, seed, tr.hit(), &vs, &ne, &missed, &cb, &cf, p);
+            if (ne.trace) sh.init(S, make_ray(ne.org, ne.dir), 0.0f, ne.tmax, lds, spill);
+        }
+        sh.template run<COUNT>(S, &c);
+        if (ne.trace) {
+            ovf = ovf || sh.st.overflow();
+            li_resolve<CACHE>(ps, ne, sh.any(), &cb);
+        }
+        if (parked) {
+            active = false;
+        } else if (active && (!more || is_zero(ps.beta))) {
+            W.L[p] = make_float4(ps.L.x, ps.L.y, ps.L.z, bitsf((uint32_t)ps.depth | (st & 0x10000u)));
+            active = false;
         }
         npool += __popcll(__ballot(parked));   // wave-uniform
         // wave-uniform: one atomic per wave for the lanes whose ray escaped
@@ -728,7 +692,7 @@ __global__ __launch_bounds__(WF_BLOCK) KPT_WPE_TAIL void k_tail(SceneView S, Fra
 }
 
 // Sky term of every path the tail ended by a miss: L + sky * beta, the same
-// operations li_bounce makes at the miss, with all lanes of a wave busy.
+// operations li_shade makes at the miss, with all lanes of a wave busy.
 __global__ __launch_bounds__(WF_BLOCK) void k_sky(FrameConst fc, WavefrontState W) {
     const int i = (int)(blockIdx.x * WF_BLOCK + threadIdx.x);
     if (i >= W.counters[cs(C_SHADOW)]) return;
@@ -760,52 +724,41 @@ __global__ __launch_bounds__(WF_BLOCK) KPT_WPE_TRACE void k_shadow(SceneView S, 
     int32_t* ctr = &W.counters[cs(pull_slot)];
     const StackShape lds{s_dyn + threadIdx.x, (int)blockDim.x, tune.stack};
     bool ovf = false;
-    if (!tune.refill) {
-        const int chunk = (tune.chunk / WAVE) * WAVE;
-        for (;;) {
-            const int base = wave_claim(ctr, chunk);
-            if (base >= count) break;
-            for (int off = 0; off < chunk && base + off < count; off += WAVE) {
-                const int kq = base + off + lane_id();
-                if (kq >= count) continue;
-                const int k = order ? order[kq] : kq;
-                const float4 o = W.shadow_o[k], d = W.shadow_d[k];
-                AnyTrav tr;
-                if (tr.init(S, make_ray(mk3(o.x, o.y, o.z), mk3(d.x, d.y, d.z)), 0.0f, o.w, lds, spill)) {
-                    while (tr.template step<false>(S, nullptr)) {}
-                }
-                ovf = ovf || tr.st.overflow;
-                shadow_resolve(W, t_lbefore, k, tr.hit);
+    // lanes take rays as in k_trace
+    const int refill_min = tune.refill ? tune.refill_min : WAVE;
+    const int chunk = max(tune.chunk / WAVE, 1) * WAVE;
+    int pos = 0, end = 0;
+    bool drained = false;
+    AnyTrav tr;
+    tr.idle();
+    int k = -1;
+    for (;;) {
+        const uint64_t m = __ballot(!tr.busy());
+        const int idle = __popcll(m);
+        if (idle >= refill_min && !(drained && pos >= end && idle < WAVE)) {
+            if (!tr.busy() && k >= 0) {
+                ovf = ovf || tr.st.overflow();
+                shadow_resolve(W, t_lbefore, k, tr.any());
+                k = -1;
             }
-        }
-    } else {
-        WaveFeeder feeder;
-        feeder.init(tune);
-        AnyTrav tr;
-        int k = -1;
-        bool busy = false;
-        for (;;) {
-            const int kk = feeder.feed(ctr, count, !busy);
-            bool done_now = false;
-            if (kk >= 0) {
-                k = order ? order[kk] : kk;
-                const float4 o = W.shadow_o[k], d = W.shadow_d[k];
-                busy = tr.init(S, make_ray(mk3(o.x, o.y, o.z), mk3(d.x, d.y, d.z)), 0.0f, o.w, lds, spill);
-                done_now = !busy;
+            if (pos >= end && !drained) {
+                const int b = wave_claim(ctr, chunk);
+                if (b >= count) drained = true;
+                else { pos = b; end = min(b + chunk, count); }
             }
-            if (!__any(busy || done_now)) {   // wave-uniform
-                if (feeder.exhausted()) break;
+            if (pos >= end) {
+                if (idle == WAVE) break;
                 continue;
             }
-            if (busy) {
-                busy = tr.template step<false>(S, nullptr);
-                done_now = !busy;
-            }
-            if (done_now) {
-                ovf = ovf || tr.st.overflow;
-                shadow_resolve(W, t_lbefore, k, tr.hit);
+            const int kq = pos + __popcll(m & lanes_below());
+            pos = min(pos + idle, end);
+            if (!tr.busy() && kq < end) {
+                k = order ? order[kq] : kq;
+                const float4 o = W.shadow_o[k], d = W.shadow_d[k];
+                tr.init(S, make_ray(mk3(o.x, o.y, o.z), mk3(d.x, d.y, d.z)), 0.0f, o.w, lds, spill);
             }
         }
+        for (int j = 0; j < TRACE_ROUNDS && __builtin_amdgcn_ballot_w64(tr.busy()) != 0ull; ++j) tr.template round<false>(S, nullptr);
     }
     if (ovf) atomicOr(overflow, 1);
 }
