@@ -298,6 +298,20 @@ KPT_HD float cosf(float x) {
     return (float)cos_d(x);
 }
 
+// sinf(x) and cosf(x), from one reduction and one evaluation of each polynomial.
+KPT_HD void sincosf(float x, float* sin_out, float* cos_out) {
+    if (f_isnan(x) || f_isinf(x) || __builtin_fabsf(x) > 1.0e6f) {
+        *sin_out = f_nan();
+        *cos_out = f_nan();
+        return;
+    }
+    int q; double r = reduce_pio2(x, &q);
+    const double sp = sin_poly(r), cp = cos_poly(r);
+    const double s = (q & 1) ? cp : sp, c = (q & 1) ? sp : cp;
+    *sin_out = (float)((q & 2) ? -s : s);
+    *cos_out = (float)(((q + 1) & 2) ? -c : c);
+}
+
 KPT_HD float tanf(float x) {
     if (f_isnan(x) || f_isinf(x)) return f_nan();
     if (__builtin_fabsf(x) > 1.0e6f) return f_nan();

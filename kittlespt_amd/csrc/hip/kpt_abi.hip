@@ -478,7 +478,7 @@ void free_frame(kpt_ctx* c) {
 void free_cache(kpt_ctx* c) {
     CacheBuffers& b = c->cb;
     dev_free(&b.w); dev_free(&b.adam_m); dev_free(&b.adam_v); dev_free(&b.grad); dev_free(&b.wb); dev_free(&b.wbt);
-    dev_free(&b.partial); dev_free(&b.partial_sum); dev_free(&b.loss_partial); dev_free(&b.stats); dev_free(&b.q_pos); dev_free(&b.q_dir);
+    dev_free(&b.partial); dev_free(&b.loss_partial); dev_free(&b.stats); dev_free(&b.q_pos); dev_free(&b.q_dir);
     dev_free(&b.q_beta); dev_free(&b.t_pos); dev_free(&b.t_dir); dev_free(&b.t_beta); dev_free(&b.t_lbefore);
     dev_free(&b.t_target); dev_free(&b.counters);
     b = CacheBuffers{};
@@ -508,7 +508,6 @@ int cache_alloc_params(kpt_ctx* ctx, int32_t batch) {
         HIPCHK(hipMalloc((void**)&b.wbt, RC_PADDED * sizeof(uint16_t)));
         HIPCHK(hipMalloc((void**)&b.stats, 4 * sizeof(float)));
         HIPCHK(hipMalloc((void**)&b.counters, 4 * sizeof(int32_t)));
-        HIPCHK(hipMalloc((void**)&b.partial_sum, (size_t)RC_CHUNKS * RC_PADDED * sizeof(float)));
         HIPCHK(hipMemsetAsync(b.grad, 0, RC_PARAMS * sizeof(float), ctx->stream));
         HIPCHK(hipMemsetAsync(b.stats, 0, 4 * sizeof(float), ctx->stream));
         HIPCHK(hipMemsetAsync(b.counters, 0, 4 * sizeof(int32_t), ctx->stream));

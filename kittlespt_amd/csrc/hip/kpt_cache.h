@@ -20,7 +20,6 @@ constexpr int RC_OUT = 3;
 constexpr int RC_LAYERS = 6;
 constexpr int RC_PARAMS = 18624;
 constexpr int RC_PADDED = 20480;
-constexpr int RC_CHUNKS = 32;    // gradient partials are summed in at most this many chunks first
 
 __host__ __device__ constexpr int rc_in(int l) { return l == 0 ? RC_IN : RC_HID; }
 __host__ __device__ constexpr int rc_out(int l) { return l == RC_LAYERS - 1 ? RC_OUT : RC_HID; }
@@ -45,7 +44,6 @@ struct CacheBuffers {
     uint16_t* wb;             // BF16 [RC_PADDED], row-major [out_pad][in] per layer
     uint16_t* wbt;            // BF16 [RC_PADDED], row-major [in][out_pad] per layer
     float* partial;           // per-workgroup gradient partials [max_wg][RC_PADDED]
-    float* partial_sum;       // sums of consecutive chunks of them [RC_CHUNKS][RC_PADDED]
     float* loss_partial;      // per-workgroup loss sums [max_wg]
     float* stats;             // [0] loss of the last step, [1] samples of the last step
     int32_t max_wg;
