@@ -283,19 +283,23 @@ KD float next_up(float x) {
 
 constexpr int INNER_RUN = 4;   // interior steps of a round
 
-// One lane's query: ANY = false the closest hit, true any hit.
-template <bool ANY>
+// One lane's query: the closest hit, any hit, or either as the lane says.
+enum TravMode : int { TRAV_CLOSEST = 0, TRAV_ANY = 1, TRAV_EITHER = 2 };
+template <int MODE>
 struct Trav {
     Ray w, o;           // the world ray; the current level's ray
     float tmin;
     float bound;        // a hit's distance has to be below this: tmax, then the closest hit so far
-    float enter;        // closest hit: a box's entry distance has to be below this
+    float enter;        // a box's entry distance has to be below this (TRAV_ANY: at most bound)
     int32_t slot, inst; // the hit (slot -1: none)
     float u, v;
     int32_t cur_inst;
     uint32_t cur;       // the entry to process next (ENTRY_IDLE: finished)
     bool fresh;         // counting: cur is a leaf that has not been counted
+    bool lane_any;      // TRAV_EITHER: this lane's query is for any hit
     LaneStack st;
+
+    KD bool is_any() const { return MODE == TRAV_ANY || (MODE == TRAV_EITHER && lane_any); }
 
     KD bool busy() const { return cur != ENTRY_IDLE; }
     KD Hit hit() const {
@@ -355,8 +359,8 @@ struct Trav {
             float c1, c2, x1, x2;
             slab_range(l1, h1, o, &c1, &x1);
             slab_range(l2, h2, o, &c2, &x2);
-            const bool k1 = c1 <= x1 && x1 >= tmin && (ANY ? c1 <= bound : c1 < enter);
-            const bool k2 = c2 <= x2 && x2 >= tmin && (ANY ? c2 <= bound : c2 < enter);
+            const bool k1 = c1 <= x1 && x1 >= tmin && (MODE == TRAV_ANY ? c1 <= bound : c1 < enter);
+            const bool k2 = c2 <= x2 && x2 >= tmin && (MODE == TRAV_ANY ? c2 <= bound : c2 < enter);
             const uint32_t e1 = bits_u(l1.w), e2 = bits_u(l2.w);
             const bool second = k2 && (!k1 || c1 > c2);
             cur = second ? e2 : e1;
@@ -424,19 +428,18 @@ struct Trav {
             const int k = __builtin_ctzll(m);
             const int to = __builtin_amdgcn_readlane(from, k) >> 2;
             const float ht = lane_of(t, k);
-            if (ANY) {
-                if (COUNT && lane == to && slot < 0) cnt->tri -= (uint32_t)((n < g ? n : g) - 1 - __builtin_amdgcn_readlane(j, k));
-                slot = lane == to ? 0 : slot;
-                cur = lane == to ? ENTRY_IDLE : cur;
-            } else {
-                const bool mine = lane == to && ht < bound;
-                slot = mine ? __builtin_amdgcn_readlane(s, k) : slot;
+            if (COUNT && lane == to && is_any() && slot < 0)   // as a lane alone would have stopped there
+                cnt->tri -= (uint32_t)((n < g ? n : g) - 1 - __builtin_amdgcn_readlane(j, k));
+            const bool mine = lane == to && ht < bound;
+            slot = mine ? __builtin_amdgcn_readlane(s, k) : slot;
+            bound = mine ? ht : bound;
+            if (MODE != TRAV_ANY) {
                 inst = mine ? cur_inst : inst;
                 u = mine ? lane_of(hu, k) : u;
                 v = mine ? lane_of(hv, k) : v;
-                bound = mine ? ht : bound;
                 enter = mine ? ht : enter;
             }
+            if (MODE != TRAV_CLOSEST) cur = mine && is_any() ? ENTRY_IDLE : cur;
         }
     }
 
@@ -448,16 +451,16 @@ struct Trav {
             load_node(S.blas_nodes, cur & ENTRY_PAYLOAD, &lo, &hi);
             if (COUNT) cnt->leaf++;
             const uint32_t first = bits_u(lo.w), n = bits_u(hi.w);
-            for (uint32_t j = 0; j < n && !(ANY && slot >= 0); ++j) {
+            for (uint32_t j = 0; j < n && !(is_any() && slot >= 0); ++j) {
                 const float4* p = reinterpret_cast<const float4*>(S.tris + first + j);
                 if (COUNT) cnt->tri++;
                 float t, hu, hv;
                 if (triangle(p[0], p[1], p[2], o.o, o.d, tmin, bound, &t, &hu, &hv)) {
                     slot = (int32_t)(first + j); inst = cur_inst; u = hu; v = hv;
-                    if (!ANY) { bound = t; enter = t; }
+                    bound = t; enter = t;
                 }
             }
-            cur = (ANY && slot >= 0) ? ENTRY_IDLE : ENTRY_POP;
+            cur = (is_any() && slot >= 0) ? ENTRY_IDLE : ENTRY_POP;
         }
     }
 
@@ -489,8 +492,9 @@ struct Trav {
         while (__builtin_amdgcn_ballot_w64(busy()) != 0ull) round<COUNT>(S, cnt);
     }
 };
-typedef Trav<false> ClosestTrav;
-typedef Trav<true> AnyTrav;
+typedef Trav<TRAV_CLOSEST> ClosestTrav;
+typedef Trav<TRAV_ANY> AnyTrav;
+typedef Trav<TRAV_EITHER> EitherTrav;
 
 // XCD-aware workgroup swizzle: the dispatcher hands consecutive workgroup ids
 // to the 8 XCDs round-robin; remap so each XCD owns a contiguous run of tiles

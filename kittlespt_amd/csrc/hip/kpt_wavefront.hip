@@ -23,11 +23,11 @@ namespace {
 constexpr int WF_BLOCK = 256;
 // Occupancy targets in waves per SIMD (512 VGPRs per lane per SIMD): the
 // traversal kernels at 8 (64 VGPRs; the closest-hit launch of a 1080p frame
-// 1.54 ms, 1.62 at 6 waves), the path-per-lane tail at 5 (96 VGPRs with the
-// path's state spilled around its traversals: 4.01 ms, 4.09 at 4 waves, 4.69
-// at 3, and 5.0 to 5.8 at 6).
+// 1.54 ms, 1.62 at 6 waves), the path-per-lane tail at 6 (80 VGPRs, the path's
+// state spilled around its rounds: 64 views 229 ms, 238 at 5 waves, 257 at 4,
+// 247 at 7 and 350 at 8).
 #define KPT_WPE_TRACE __attribute__((amdgpu_waves_per_eu(8)))
-#define KPT_WPE_TAIL __attribute__((amdgpu_waves_per_eu(5)))
+#define KPT_WPE_TAIL __attribute__((amdgpu_waves_per_eu(6)))
 constexpr int TRACE_ROUNDS = 8;   // traversal rounds of a wave between looks at its idle lanes
 constexpr int MAX_KEYS = 64;
 // counters[] slots (zeroed once per frame by a fill kernel)
@@ -500,7 +500,8 @@ constexpr int TAIL_SLOT_HEAD = 4;     // float4 of a parked trace's state before
 constexpr int TAIL_SAVE_STACK = 48;   // stack entries a parked trace may hold
 constexpr int TAIL_SLOT_F4 = TAIL_SLOT_HEAD + TAIL_SAVE_STACK / 4;   // float4 per parked trace
 static_assert(TAIL_POOL * TAIL_SLOT_F4 * 16 == TAIL_POOL_BYTES, "pool layout");
-constexpr int TAIL_CHECK = 32;        // traversal rounds between parking checks
+constexpr int TAIL_CHECK = 8;       // traversal rounds between looks at the lanes that have ended
+constexpr int TAIL_SWITCH = 16;      // lanes with an ended shadow ray that the wave stops for
 
 template <bool COUNT, bool CACHE>
 __global__ __launch_bounds__(WF_BLOCK) KPT_WPE_TAIL void k_tail(SceneView S, FrameConst fc, WavefrontState W, int parity,
@@ -518,6 +519,11 @@ __global__ __launch_bounds__(WF_BLOCK) KPT_WPE_TAIL void k_tail(SceneView S, Fra
     int npool = 0;   // wave-uniform: parked traces in the wave's slots [0, npool)
     bool ovf = false;
     bool active = false, drained = false;   // drained: wave-uniform
+    bool more = false;      // the path goes on: its ray (ps.ray) has a closest-hit trace to make
+    bool shadow = false;    // the lane's query is the previous vertex's shadow ray
+    bool pend = false, occluded = false;   // that ray has ended, its term not yet added to L
+    NeeResult ne;           // the previous vertex's estimate
+    ne.trace = false;
     int p = -1;
     uint32_t st = 0u, seed = 0u;
     PathState ps;
@@ -570,54 +576,82 @@ __global__ __launch_bounds__(WF_BLOCK) KPT_WPE_TAIL void k_tail(SceneView S, Fra
             if (COUNT && W.heat) heat_px = W.heat + 2 * (int64_t)fbits(o4.w);
         }
         if (!__any(active)) break;   // wave-uniform: queue drained, nothing parked, every lane idle
-        // the vertex's closest-hit trace: begun here, or taken back where it was
-        // parked.  All lanes go through the traversals, with or without a query
-        // of their own: the triangles of a leaf are spread over the wave.
+        // A vertex's shadow ray and its continuation's closest-hit trace do not
+        // depend on one another: a lane traces the one, then the other, and the
+        // wave waits for its lanes once a vertex instead of twice (8-spp 1080p
+        // frames 48.4 -> 45.2 ms, 64 views 251 -> 229 ms; switching at 8, 16 and
+        // 32 ended shadow rays measured alike).  All lanes go through the rounds, with or without a query of their own: the
+        // triangles of a leaf are spread over the wave.
         bool missed = false, parked = false;
-        const bool tracing = active && (resumed || !is_zero(ps.beta));
-        ClosestTrav tr;
+        EitherTrav tr;
         tr.idle();
-        if (tracing) {
-            if (resumed) {
-                // the world ray is the path's ray (as the trace was begun with it), the
-                // object ray recomputed from it as the instance step computed it
-                const float4* sl = pool + slot * TAIL_SLOT_F4;
-                const float4 a0 = sl[0], a1 = sl[1], a2 = sl[2], a3 = sl[3];
-                tr.w = ps.ray;
-                tr.tmin = a0.y; tr.bound = a0.z; tr.enter = a0.w;
-                tr.slot = (int32_t)fbits(a1.x); tr.inst = (int32_t)fbits(a1.y); tr.u = a1.z; tr.v = a1.w;
-                tr.cur_inst = (int32_t)fbits(a2.x); tr.cur = fbits(a2.y); tr.fresh = fbits(a2.z) != 0u;
-                const int sp = (int)fbits(a3.x);
-                tr.o = (tr.cur & TLAS_BIT) ? tr.w : object_ray(S.inst_trav[tr.cur_inst], tr.w);
-                tr.st.reset(lds, spill);
-                for (int i = 0; i < sp; i += 4) {
-                    const float4 e = sl[TAIL_SLOT_HEAD + i / 4];
-                    tr.st.push(fbits(e.x));
-                    if (i + 1 < sp) tr.st.push(fbits(e.y));
-                    if (i + 2 < sp) tr.st.push(fbits(e.z));
-                    if (i + 3 < sp) tr.st.push(fbits(e.w));
-                }
-            } else {
-                if (COUNT) ++n_vertices;
-                seed = seed + (uint32_t)ps.depth;
-                tr.init(S, ps.ray, 0.0f, __builtin_inff(), lds, spill);
+        uint32_t b0 = 0u, t0 = 0u;   // counting mode: the lane's counts when its closest-hit trace began
+        auto closest = [&]() {
+            if (COUNT) { ++n_vertices; b0 = c.interior + c.leaf; t0 = c.tlas; }
+            seed = seed + (uint32_t)ps.depth;
+            tr.init(S, ps.ray, 0.0f, __builtin_inff(), lds, spill);
+            tr.lane_any = false;
+        };
+        if (fresh || resumed) more = resumed || !is_zero(ps.beta);
+        shadow = active && !fresh && !resumed && ne.trace;
+        if (resumed) {
+            // the world ray is the path's ray (as the trace was begun with it), the
+            // object ray recomputed from it as the instance step computed it
+            if (COUNT) { b0 = c.interior + c.leaf; t0 = c.tlas; }
+            const float4* sl = pool + slot * TAIL_SLOT_F4;
+            const float4 a0 = sl[0], a1 = sl[1], a2 = sl[2], a3 = sl[3];
+            tr.w = ps.ray;
+            tr.lane_any = false;
+            tr.tmin = a0.y; tr.bound = a0.z; tr.enter = a0.w;
+            tr.slot = (int32_t)fbits(a1.x); tr.inst = (int32_t)fbits(a1.y); tr.u = a1.z; tr.v = a1.w;
+            tr.cur_inst = (int32_t)fbits(a2.x); tr.cur = fbits(a2.y); tr.fresh = fbits(a2.z) != 0u;
+            const int sp = (int)fbits(a3.x);
+            tr.o = (tr.cur & TLAS_BIT) ? tr.w : object_ray(S.inst_trav[tr.cur_inst], tr.w);
+            tr.st.reset(lds, spill);
+            for (int i = 0; i < sp; i += 4) {
+                const float4 e = sl[TAIL_SLOT_HEAD + i / 4];
+                tr.st.push(fbits(e.x));
+                if (i + 1 < sp) tr.st.push(fbits(e.y));
+                if (i + 2 < sp) tr.st.push(fbits(e.z));
+                if (i + 3 < sp) tr.st.push(fbits(e.w));
             }
+        } else if (shadow) {
+            tr.init(S, make_ray(ne.org, ne.dir), 0.0f, ne.tmax, lds, spill);
+            tr.lane_any = true;
+        } else if (active && more) {
+            closest();
         }
-        const uint32_t b0 = COUNT ? c.interior + c.leaf : 0u, t0 = COUNT ? c.tlas : 0u;
-        // TAIL_CHECK rounds between looks at how many lanes still trace
+        // TAIL_CHECK rounds between looks at the lanes that have ended
         uint64_t mp = 0ull;   // the traces to park
         for (;;) {
             for (int j = 0; j < TAIL_CHECK && __builtin_amdgcn_ballot_w64(tr.busy()) != 0ull; ++j)
                 tr.template round<COUNT>(S, &c);
             mp = __ballot(tr.busy());
+            const bool ended = shadow && !tr.busy();
+            const uint64_t me = __ballot(ended);
+            if (me != 0ull && (__popcll(me) >= TAIL_SWITCH || mp == 0ull)) {
+                if (ended) {
+                    ovf = ovf || tr.st.overflow();
+                    occluded = tr.any();
+                    pend = true;
+                    shadow = false;
+                    tr.idle();
+                    if (more) closest();
+                }
+                continue;
+            }
             if (mp == 0ull) break;
-            if (pool && !drained && __popcll(mp) < suspend && __popcll(mp) <= TAIL_POOL - npool &&
-                __ballot(tr.busy() && tr.st.size() > TAIL_SAVE_STACK) == 0ull)
+            if (pool && !drained && me == 0ull && __popcll(mp) < suspend && __popcll(mp) <= TAIL_POOL - npool &&
+                __ballot(tr.busy() && (shadow || tr.st.size() > TAIL_SAVE_STACK)) == 0ull)
                 break;
         }
-        if (COUNT && heat_px && tracing) {
+        if (COUNT && heat_px && active && more) {
             atomicAdd(&heat_px[0], (int32_t)(c.interior + c.leaf - b0));
             atomicAdd(&heat_px[1], (int32_t)(c.tlas - t0));
+        }
+        if (pend) {
+            li_resolve<CACHE>(ps, ne, occluded, &cb);
+            pend = false;
         }
         // the traces still running are parked in the wave's slots from npool on
         if (tr.busy()) {
@@ -645,27 +679,19 @@ __global__ __launch_bounds__(WF_BLOCK) KPT_WPE_TAIL void k_tail(SceneView S, Fra
             }
             parked = true;
         }
-        // shading, then the wave's shadow rays
-        bool more = false;
-        NeeResult ne;
-        ne.trace = false;
-        AnyTrav sh;
-        sh.idle();
-        if (tracing && !parked) {
-            ovf = ovf || tr.st.overflow();
-            more = li_shade<true, CACHE>(S, fc, ps, seed, tr.hit(), &vs, &ne, &missed, &cb, &cf, p);
-            if (ne.trace) sh.init(S, make_ray(ne.org, ne.dir), 0.0f, ne.tmax, lds, spill);
-        }
-        sh.template run<COUNT>(S, &c);
-        if (ne.trace) {
-            ovf = ovf || sh.st.overflow();
-            li_resolve<CACHE>(ps, ne, sh.any(), &cb);
-        }
         if (parked) {
             active = false;
-        } else if (active && (!more || is_zero(ps.beta))) {
-            W.L[p] = make_float4(ps.L.x, ps.L.y, ps.L.z, bitsf((uint32_t)ps.depth | (st & 0x10000u)));
-            active = false;
+        } else if (active) {
+            ne.trace = false;
+            if (more) {
+                ovf = ovf || tr.st.overflow();
+                more = li_shade<true, CACHE>(S, fc, ps, seed, tr.hit(), &vs, &ne, &missed, &cb, &cf, p) &&
+                       !is_zero(ps.beta);
+            }
+            if (!more && !ne.trace) {
+                W.L[p] = make_float4(ps.L.x, ps.L.y, ps.L.z, bitsf((uint32_t)ps.depth | (st & 0x10000u)));
+                active = false;
+            }
         }
         npool += __popcll(__ballot(parked));   // wave-uniform
         // wave-uniform: one atomic per wave for the lanes whose ray escaped
