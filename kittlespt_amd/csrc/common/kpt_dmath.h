@@ -75,6 +75,21 @@ KPT_HD double scaled(double x, int n) {
 #define KPT_LN2_LO 1.42860682030941723212e-6f
 #define KPT_LOG2E 1.44269504088896340736f
 
+// e^x for |x| < 87, where 2^k is a normal float.
+KPT_HD float expf_normal(float x) {
+    float k = __builtin_rintf(x * KPT_LOG2E);
+    float r = (x - k * KPT_LN2_HI) - k * KPT_LN2_LO;
+    float p = (float)(1.0 / 5040.0);
+    p = p * r + (float)(1.0 / 720.0);
+    p = p * r + (float)(1.0 / 120.0);
+    p = p * r + (float)(1.0 / 24.0);
+    p = p * r + (float)(1.0 / 6.0);
+    p = p * r + 0.5f;
+    p = p * r + 1.0f;
+    p = p * r + 1.0f;
+    return p * pow2f((int)k);
+}
+
 KPT_HD float expf(float x) {
     if (f_isnan(x)) return x;
     if (x > 88.7228394f) return f_inf();
