@@ -327,6 +327,9 @@ KD void li_resolve(PathState& ps, const NeeResult& ne, bool occluded, const Cach
     if (CACHE && ne.trec >= 0) cb->t_lbefore[ne.trec] = make_float4(ps.L.x, ps.L.y, ps.L.z, 0.0f);
 }
 
+constexpr int MEGA_CHECK = 8;     // traversal rounds between looks at the lanes that have ended
+constexpr int MEGA_SWITCH = 16;   // lanes with an ended shadow ray that the wave stops for
+
 // Megakernel form of Li: the whole path in one thread, the wave's lanes
 // vertex by vertex together (all of them call; live: the lane has a path).
 __device__ __forceinline__ v3 li_path(const SceneView& S, const FrameConst& fc, bool live, Ray ray, uint32_t& seed,
@@ -340,27 +343,51 @@ __device__ __forceinline__ v3 li_path(const SceneView& S, const FrameConst& fc, 
     ps.p_b = 1.0f;
     ps.prev_pos = mk3(0.0f, 0.0f, 0.0f);
     uint32_t spill[SPILL_STACK];
+    // a lane traces a vertex's shadow ray, then its continuation (as the
+    // wavefront's tail does): the wave waits for its lanes once a vertex
+    bool more = live;         // the path goes on: ps.ray has a closest-hit trace to make
+    NeeResult ne;             // the previous vertex's estimate
+    ne.trace = false;
     while (__builtin_amdgcn_ballot_w64(live) != 0ull) {
-        ClosestTrav tr;
+        EitherTrav tr;
         tr.idle();
-        if (live) {
+        bool shadow = live && ne.trace, pend = false, occluded = false;
+        auto closest = [&]() {
             seed = seed + (uint32_t)ps.depth;
             tr.init(S, ps.ray, 0.0f, __builtin_inff(), lds, spill);
+            tr.lane_any = false;
+        };
+        if (shadow) {
+            tr.init(S, make_ray(ne.org, ne.dir), 0.0f, ne.tmax, lds, spill);
+            tr.lane_any = true;
+        } else if (live && more) {
+            closest();
         }
-        tr.template run<false>(S, nullptr);
-        NeeResult ne;
+        for (;;) {
+            for (int j = 0; j < MEGA_CHECK && __builtin_amdgcn_ballot_w64(tr.busy()) != 0ull; ++j)
+                tr.template round<false>(S, nullptr);
+            const bool ended = shadow && !tr.busy();
+            const uint64_t me = __builtin_amdgcn_ballot_w64(ended), mb = __builtin_amdgcn_ballot_w64(tr.busy());
+            if (me == 0ull && mb == 0ull) break;
+            if (me != 0ull && (__builtin_popcountll(me) >= MEGA_SWITCH || mb == 0ull)) {
+                if (ended) {
+                    *ovf = *ovf || tr.st.overflow();
+                    occluded = tr.any();
+                    pend = true;
+                    shadow = false;
+                    tr.idle();
+                    if (more) closest();
+                }
+            }
+        }
+        if (pend) li_resolve(ps, ne, occluded);
         ne.trace = false;
-        AnyTrav sh;
-        sh.idle();
         if (live) {
-            *ovf = *ovf || tr.st.overflow();
-            live = li_shade(S, fc, ps, seed, tr.hit(), vs, &ne) && !is_zero(ps.beta);
-            if (ne.trace) sh.init(S, make_ray(ne.org, ne.dir), 0.0f, ne.tmax, lds, spill);
-        }
-        sh.template run<false>(S, nullptr);
-        if (ne.trace) {
-            *ovf = *ovf || sh.st.overflow();
-            li_resolve(ps, ne, sh.any());
+            if (more) {
+                *ovf = *ovf || tr.st.overflow();
+                more = li_shade(S, fc, ps, seed, tr.hit(), vs, &ne) && !is_zero(ps.beta);
+            }
+            live = more || ne.trace;
         }
     }
     return ps.L;

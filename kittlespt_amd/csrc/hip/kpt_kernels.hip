@@ -100,8 +100,8 @@ hipError_t launch_trace_any(hipStream_t s, const SceneView& S, const kpt_ray* ra
 // accumulation (Integrator::addSample, integrator.cuh:406-416) or temporal
 // reprojection (reprojectAccumulate, kernels.cu:299-338).  16x16 pixel
 // tiles, XCD-swizzled tile order.  4 waves per SIMD (128 VGPRs): a 640x360
-// frame of depth 3 takes 1066 us, 1157 at 3 waves, 1273 unconstrained (207
-// VGPRs), 1159 at 5.
+// frame of depth 3 takes 937 us, 1017 at 3 waves, 983 at 5, 996 at 6 (1067 at
+// 4 with the shadow rays traced before the next vertex's rays, wave by wave).
 constexpr int TILE = 16;
 
 __global__ __launch_bounds__(TRACE_BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void k_megakernel(SceneView S, FrameConst fc, int32_t frame,
