@@ -1573,7 +1573,7 @@ int kpt_render(kpt_ctx* ctx, int32_t spp) {
                 if (graph) tune.ray_sort = 0;
                 e = wavefront_frame(fs, S, fc, ctx->frame_index, ctx->fb, fw, ctx->d_overflow,
                                     (int32_t)ctx->materials.size(), ctx->sort_by_material, tune, ins,
-                                    use_cache ? &hooks : nullptr, nullptr, prev_done);
+                                    use_cache ? &hooks : nullptr, nullptr, prev_done, overlap);
                 if (e != hipSuccess) return e;
                 if (use_cache && cs.train) {
                     // Adam steps over this frame's suffixes (they shape the next frames)

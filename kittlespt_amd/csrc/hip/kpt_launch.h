@@ -220,11 +220,13 @@ hipError_t launch_heat_colour(hipStream_t s, const int32_t* heat, int64_t n, flo
 // or writes the cache (its bounce-1 work: the cache vertex is never the
 // primary one), and starts its cache frame there, so that its records,
 // queries and inference follow the previous frame's training.
+// two_in_flight: another frame's stages run beside this one's (a choice of
+// launches depends on it, results do not).
 hipError_t wavefront_frame(hipStream_t s, const SceneView& S, const FrameConst& fc, int32_t frame,
                            const FrameBuffers& fb, WavefrontState& W, int32_t* overflow, int32_t num_materials,
                            int32_t sort_by_material, const TraceTuning& tune, WfInstrument* ins,
                            const CacheHooks* cache, const ViewBatch* views = nullptr,
-                           hipEvent_t finish_after = nullptr);
+                           hipEvent_t finish_after = nullptr, bool two_in_flight = false);
 
 // Radiance-cache kernels (kpt_cache.hip).
 int cache_train_workgroups(int32_t batch);

@@ -42,6 +42,12 @@ static_assert(C_PULL + 3 * MAX_BOUNCE_SLOTS <= WF_COUNTER_SLOTS, "counter slots"
 // channels instead of queueing behind one another on one line.
 KD int cs(int slot) { return slot * WF_COUNTER_STRIDE; }
 
+// Flags in W.L's w above the depth (bits 0..15) and li_shade's own (16..18): a
+// path queued for the tail with its vertex's shadow ray still to trace, and
+// one queued for that ray alone.
+constexpr uint32_t ST_SHADOW = 0x80000u;
+constexpr uint32_t ST_ENDED = 0x100000u;
+
 KD uint32_t fbits(float f) { return __builtin_bit_cast(uint32_t, f); }
 KD float bitsf(uint32_t u) { return __builtin_bit_cast(float, u); }
 
@@ -333,8 +339,11 @@ __global__ __launch_bounds__(WF_BLOCK) void k_sort_scatter(SceneView S, Wavefron
 // its waves' ballots in LDS): the appends of every workgroup target the same
 // two counters, and one atomic per 256 lanes instead of one per wave and
 // queue keeps that address's queue in L2 short.
+// to_tail: the next bounce is the tail's.  Shadow rays are then not queued for
+// a launch of their own: each stays with its path (ended paths with one are
+// queued too), whose lane of the tail traces it first.
 __global__ __launch_bounds__(WF_BLOCK) void k_shade(SceneView S, FrameConst fc, WavefrontState W, int parity,
-                                                    const int32_t* q, CacheBuffers cb, CacheFrame cf) {
+                                                    const int32_t* q, CacheBuffers cb, CacheFrame cf, int to_tail) {
     constexpr int NW = WF_BLOCK / WAVE;
     __shared__ int s_off[2][NW + 1];   // per queue: the waves' offsets, then the workgroup's base
     const int count = W.counters[cs(C_QCOUNT + parity)];
@@ -434,12 +443,22 @@ __global__ __launch_bounds__(WF_BLOCK) void k_shade(SceneView S, FrameConst fc, 
                 }
             }
         }
+        const bool with_tail = want_shadow && to_tail != 0;
         W.L[p] = make_float4(L.x, L.y, L.z, bitsf((uint32_t)depth | (any_nonspec ? 0x10000u : 0u) |
-                                                  (wide_in ? 0x20000u : 0u) | (cached ? 0x40000u : 0u)));
+                                                  (wide_in ? 0x20000u : 0u) | (cached ? 0x40000u : 0u) |
+                                                  (with_tail ? ST_SHADOW | (alive ? 0u : ST_ENDED) : 0u)));
         W.ray_d[p] = make_float4(ray.d.x, ray.d.y, ray.d.z, bitsf(seed));
         if (alive) {
             W.ray_o[p] = make_float4(ray.o.x, ray.o.y, ray.o.z, o4.w);
             W.beta[p] = make_float4(beta.x, beta.y, beta.z, p_b);
+        }
+        if (with_tail) {   // by path, for the tail
+            W.shadow_o[p] = sh_o;
+            W.shadow_d[p] = sh_d;
+            W.shadow_c[p] = sh_c;
+            W.shadow_z[p] = sh_z;
+            alive = true;
+            want_shadow = false;
         }
     }
     const uint64_t m_sh = __ballot(want_shadow), m_al = __ballot(alive);
@@ -478,10 +497,11 @@ __global__ __launch_bounds__(WF_BLOCK) void k_shade(SceneView S, FrameConst fc, 
 // numbers as the stage kernels, so the radiance is unchanged.  Lanes refill
 // at vertex boundaries: a lane whose path ends takes the next queued path
 // before the wave's next vertex, so a wave is not held by its longest path.
-// A path whose ray escapes leaves its sky term to k_sky: the lane appends
-// (path, direction, throughput) to the sky queue (the shadow-ray arrays,
-// unused while the tail runs; count in C_SHADOW, cleared before the launch)
-// instead of evaluating the sky with the few lanes that missed.
+// A path whose ray escapes leaves its sky term to k_sky: the lane leaves its
+// direction and throughput in the path's arrays and appends the path to the
+// sky queue (W.sort_tmp, unused while the tail runs; count in C_SHADOW, cleared
+// before the launch) instead of evaluating the sky with the few lanes that
+// missed.
 // Parked traces (suspend > 0): a vertex's closest-hit trace holds the whole
 // wave until its longest ray ends, while most lanes have finished.  Once
 // fewer than `suspend` lanes are still tracing (and the wave can still claim
@@ -574,6 +594,16 @@ __global__ __launch_bounds__(WF_BLOCK) KPT_WPE_TAIL void k_tail(SceneView S, Fra
             seed = fbits(d4.w);
             active = true;
             if (COUNT && W.heat) heat_px = W.heat + 2 * (int64_t)fbits(o4.w);
+            ne.trace = fresh && (st & ST_SHADOW);
+            if (ne.trace) {   // the estimate of the vertex before, left to the tail
+                const float4 so = W.shadow_o[p], sd = W.shadow_d[p], sc = W.shadow_c[p], sz = W.shadow_z[p];
+                ne.org = mk3(so.x, so.y, so.z);
+                ne.tmax = so.w;
+                ne.dir = mk3(sd.x, sd.y, sd.z);
+                ne.trec = (int32_t)fbits(sd.w);
+                ne.unoccl = mk3(sc.x, sc.y, sc.z);
+                ne.occl = mk3(sz.x, sz.y, sz.z);
+            }
         }
         if (!__any(active)) break;   // wave-uniform: queue drained, nothing parked, every lane idle
         // A vertex's shadow ray and its continuation's closest-hit trace do not
@@ -592,8 +622,8 @@ __global__ __launch_bounds__(WF_BLOCK) KPT_WPE_TAIL void k_tail(SceneView S, Fra
             tr.init(S, ps.ray, 0.0f, __builtin_inff(), lds, spill);
             tr.lane_any = false;
         };
-        if (fresh || resumed) more = resumed || !is_zero(ps.beta);
-        shadow = active && !fresh && !resumed && ne.trace;
+        if (fresh || resumed) more = resumed || (!(st & ST_ENDED) && !is_zero(ps.beta));
+        shadow = active && ne.trace;
         if (resumed) {
             // the world ray is the path's ray (as the trace was begun with it), the
             // object ray recomputed from it as the instance step computed it
@@ -700,9 +730,9 @@ __global__ __launch_bounds__(WF_BLOCK) KPT_WPE_TAIL void k_tail(SceneView S, Fra
             const int base = wave_claim(&W.counters[cs(C_SHADOW)], __popcll(mm));
             if (missed) {
                 const int k = base + __popcll(mm & lanes_below());
-                W.shadow_queue[k] = p;
-                W.shadow_d[k] = make_float4(ps.ray.d.x, ps.ray.d.y, ps.ray.d.z, 0.0f);
-                W.shadow_c[k] = make_float4(ps.beta.x, ps.beta.y, ps.beta.z, 0.0f);
+                W.sort_tmp[k] = p;
+                W.ray_d[p] = make_float4(ps.ray.d.x, ps.ray.d.y, ps.ray.d.z, bitsf(seed));
+                W.beta[p] = make_float4(ps.beta.x, ps.beta.y, ps.beta.z, ps.p_b);
             }
         }
     }
@@ -722,8 +752,8 @@ __global__ __launch_bounds__(WF_BLOCK) KPT_WPE_TAIL void k_tail(SceneView S, Fra
 __global__ __launch_bounds__(WF_BLOCK) void k_sky(FrameConst fc, WavefrontState W) {
     const int i = (int)(blockIdx.x * WF_BLOCK + threadIdx.x);
     if (i >= W.counters[cs(C_SHADOW)]) return;
-    const int p = W.shadow_queue[i];
-    const float4 d = W.shadow_d[i], b = W.shadow_c[i], l = W.L[p];
+    const int p = W.sort_tmp[i];
+    const float4 d = W.ray_d[p], b = W.beta[p], l = W.L[p];
     const v3 sky = miss_radiance(fc, mk3(d.x, d.y, d.z), false);
     const v3 L = mk3(l.x, l.y, l.z) + sky * mk3(b.x, b.y, b.z);
     W.L[p] = make_float4(L.x, L.y, L.z, l.w);
@@ -806,12 +836,18 @@ __global__ __launch_bounds__(WF_BLOCK) void k_finish(SceneView S, FrameConst fc,
 
 int g_num_cus = 0;
 
+// Frames up to this many pixels leave the shadow rays of the bounce before the
+// tail to it: alone on the GPU and without the cache, and otherwise
+// (wavefront_frame has both sides measured).
+constexpr int64_t SHADOW_TAIL_PX1 = 1 << 21;
+constexpr int64_t SHADOW_TAIL_PX2 = 1 << 19;
+
 }  // namespace
 
 hipError_t wavefront_frame(hipStream_t s, const SceneView& S, const FrameConst& fc, int32_t frame,
                            const FrameBuffers& fb, WavefrontState& W, int32_t* overflow, int32_t num_materials,
                            int32_t sort_by_material, const TraceTuning& tune, WfInstrument* ins,
-                           const CacheHooks* cache, const ViewBatch* views, hipEvent_t finish_after) {
+                           const CacheHooks* cache, const ViewBatch* views, hipEvent_t finish_after, bool two_in_flight) {
     if (ins) {
         ins->launches = 0;
         ins->tail_launches = 0;
@@ -955,13 +991,25 @@ hipError_t wavefront_frame(hipStream_t s, const SceneView& S, const FrameConst& 
             hipLaunchKernelGGL(k_sort_scatter, dim3(pgrid), dim3(WF_BLOCK), 0, s, S, W, parity, nkeys);
             shade_q = W.sort_tmp;
         }
+        // The last bounce before the tail leaves its shadow rays to it on frames
+        // small enough that one launch and its drain less outweighs their slower
+        // traversal there (80 registers of mixed queries against 64): with one
+        // frame on the GPU 9 % at 320x180, 7 % at 960x540, 2 % at 1920x1080 (1000
+        // instances; 9, 14 and 5 % on one object); with two, whose stages fill each
+        // other's drains, 8 % at 320x180, 1 % at 960x540, and 2 to 5 % slower above
+        // a million pixels; with the cache, whose ended paths are most of that bounce's,
+        // 2 % slower at 1920x1080.  Counted frames keep them apart from the tail's events.
+        const int to_tail = tune.tail > 0 && bounce + 1 >= tune.tail && bounce + 1 < max_bounces &&
+                            npx <= (two_in_flight || cache ? SHADOW_TAIL_PX2 : SHADOW_TAIL_PX1) && !(ins && ins->counters);
         const bool time_shade = ins && bounce == 0;
         if (time_shade) (void)hipEventRecord(ins->xbegin[WF_X_SHADE0], s);
-        hipLaunchKernelGGL(k_shade, dim3(gblocks), dim3(WF_BLOCK), 0, s, S, fc, W, parity, shade_q, cb, cf);
+        hipLaunchKernelGGL(k_shade, dim3(gblocks), dim3(WF_BLOCK), 0, s, S, fc, W, parity, shade_q, cb, cf,
+                           to_tail);
         if (time_shade) {
             (void)hipEventRecord(ins->xend[WF_X_SHADE0], s);
             ins->xlaunches[WF_X_SHADE0] = 1;
         }
+        if (to_tail) continue;
         const int32_t* shadow_order = nullptr;
         if (tune.ray_sort && W.rtemp) {
             hipLaunchKernelGGL(k_shadow_keys, dim3(gblocks), dim3(WF_BLOCK), 0, s, fc, W, npx);
