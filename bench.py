@@ -740,7 +740,7 @@ def main():
             avg_s = cache_acc["cache_train_ms"] / cache_acc["cache_train_launches"] / 1e3
             used = cache_acc["trained"] / nf
             fl = used * MLP_TRAIN_FLOP
-            mlp["train"] = {"kernel": "k_rc_train + k_rc_reduce + k_rc_adam (4 Adam steps per frame)",
+            mlp["train"] = {"kernel": "k_rc_train + k_rc_adam (4 Adam steps per frame)",
                             "bound": "mfma", "unit": "TFLOP/s", "achieved": round(fl / avg_s / 1e12, 3),
                             "peak": MFMA_PEAK_TFLOPS, "frac": round(fl / avg_s / 1e12 / MFMA_PEAK_TFLOPS, 5),
                             "samples_per_frame": int(used), "flop_per_frame": int(fl),
