@@ -58,3 +58,46 @@ def test_knobs(ctx, knobs):
     finally:
         c.set_tuning(**keep)
     assert np.array_equal(got, want)
+
+
+@pytest.fixture(scope="module")
+def instanced():
+    c = Context(0)
+    sc = scenes.scene_instanced_small()
+    c.upload(sc)
+    yield sc, c
+    c.close()
+
+
+@pytest.mark.parametrize("W,H,spp", ((67, 45, 1), (67, 45, 3), (1024, 512, 2), (1024, 513, 2), (2048, 1024, 1),
+                                     (2048, 1025, 1)))
+@pytest.mark.parametrize("tail", (1, 2))
+def test_instances_equal_the_megakernel(instanced, W, H, spp, tail):
+    sc, c = instanced
+    print(f"[shadow tail] instances, {W}x{H}, {spp} spp, tail {tail}", flush=True)
+    want = image(sc, c, W, H, abi.INTEGRATOR_MEGAKERNEL, 4, spp)
+    got = image(sc, c, W, H, abi.INTEGRATOR_WAVEFRONT, 4, spp, tail=tail)
+    assert np.array_equal(got, want)
+
+
+# the rule goes by the batch's pixels: 3 x 64 x 48, and 2^21 of them and 2048 more
+@pytest.mark.parametrize("sizes", (((64, 48), (37, 29), (1, 1)), ((1024, 1024), (512, 2048)),
+                                   ((1024, 1024), (512, 2048), (64, 32))))
+@pytest.mark.parametrize("tail", (1, 2))
+def test_view_batches(instanced, sizes, tail):
+    sc, c = instanced
+    eye, to = np.array(sc.camera_eye, np.float64), np.array(sc.camera_target, np.float64)
+    views = [(scenes.perspective_fov_lh(sc.camera_fov, w, h, 1.0, 100.0),
+              scenes.look_at_view(eye * (1 + 0.1 * k), to), w, h) for k, (w, h) in enumerate(sizes)]
+    c.set_settings(settings(max_depth=5, integrator=abi.INTEGRATOR_WAVEFRONT, sun_theta=sc.sun_theta))
+    keep = c.tuning()
+    try:
+        got = {}
+        for t in (0, tail):
+            print(f"[shadow tail] views {sizes}, tail {t}", flush=True)
+            c.set_tuning(tail=t, graph=0, ray_sort=0)
+            got[t] = c.render_views(views, spp=2)
+    finally:
+        c.set_tuning(**keep)
+    for a, b in zip(got[0], got[tail]):
+        assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
