@@ -836,11 +836,34 @@ __global__ __launch_bounds__(WF_BLOCK) void k_finish(SceneView S, FrameConst fc,
 
 int g_num_cus = 0;
 
-// Frames up to this many pixels leave the shadow rays of the bounce before the
-// tail to it: alone on the GPU and without the cache, and otherwise
-// (wavefront_frame has both sides measured).
-constexpr int64_t SHADOW_TAIL_PX1 = 1 << 21;
-constexpr int64_t SHADOW_TAIL_PX2 = 1 << 19;
+// Whether a frame's (or a view batch's) last bounce before the tail leaves its
+// shadow rays to the tail: one launch and its drain less, against a slower
+// traversal there (80 registers of mixed queries against 64).  Time of a frame
+// with the separate launch over the time with them in the tail, 1000 instances
+// (one object), 2^12 to 2^23 pixels, depth 8 (4):
+//   pixels                    2^12  2^15  2^17  2^18  2^19  2^20  2^20.5 2^21  2^22  2^23
+//   one frame                 1.07  1.09  1.10  1.09  1.08  1.04  1.03   1.02  0.99  0.98
+//                            (1.09  1.10  1.10  1.11  1.13  1.10  1.07   1.06  1.02  1.01)
+//   one, cached and trained   1.08  1.07  1.09  1.13  1.12  1.04  1.03   1.02  1.00  0.98
+//                            (1.09  1.09  1.07  1.08  1.08  1.06  1.03   1.02  1.00  0.98)
+//   one batch of 8 views         -     -     -  1.10  1.06  1.03     -   1.02  1.00  0.98
+//                            (   -     -     -  1.10  1.13  1.08     -   1.05  1.02  1.01)
+//   two frames in flight      1.05  1.06  1.08  1.07  1.01  0.96  0.95   0.96  0.98  0.97
+//                            (1.08  1.08  1.11  1.14  1.07  1.08  1.04   0.97  0.99  0.99)
+//   two, cached and trained   0.96  0.97  0.99  1.03  1.07  0.98  0.98   0.98  0.98  0.96
+//                            (1.03  1.02  1.02  1.03  1.04  1.05  1.00   0.99  0.98  0.98)
+//   two, cached               0.90  0.95  0.97  0.99  1.05  0.97  0.94   0.94     -     -
+//                            (0.95  0.91  0.99  1.04  1.11  1.07  1.04   1.02     -     -)
+// Two frames fill each other's drains, so the line lies lower; and a cached
+// frame's tail waits for the previous frame while its own bounce 0, with a
+// launch for the shadow rays, does not: small ones are better off with it.
+constexpr int64_t SHADOW_TAIL_ONE = 1 << 21;
+constexpr int64_t SHADOW_TAIL_TWO = 1 << 19;
+constexpr int64_t SHADOW_TAIL_TWO_CACHED_FROM = 1 << 18;
+bool shadows_to_tail(int64_t npx, bool two_in_flight, bool cached) {
+    if (!two_in_flight) return npx <= SHADOW_TAIL_ONE;
+    return npx <= SHADOW_TAIL_TWO && (!cached || npx >= SHADOW_TAIL_TWO_CACHED_FROM);
+}
 
 }  // namespace
 
@@ -991,16 +1014,9 @@ hipError_t wavefront_frame(hipStream_t s, const SceneView& S, const FrameConst& 
             hipLaunchKernelGGL(k_sort_scatter, dim3(pgrid), dim3(WF_BLOCK), 0, s, S, W, parity, nkeys);
             shade_q = W.sort_tmp;
         }
-        // The last bounce before the tail leaves its shadow rays to it on frames
-        // small enough that one launch and its drain less outweighs their slower
-        // traversal there (80 registers of mixed queries against 64): with one
-        // frame on the GPU 9 % at 320x180, 7 % at 960x540, 2 % at 1920x1080 (1000
-        // instances; 9, 14 and 5 % on one object); with two, whose stages fill each
-        // other's drains, 8 % at 320x180, 1 % at 960x540, and 2 to 5 % slower above
-        // a million pixels; with the cache, whose ended paths are most of that bounce's,
-        // 2 % slower at 1920x1080.  Counted frames keep them apart from the tail's events.
+        // (counted frames keep the shadow rays apart from the tail's events)
         const int to_tail = tune.tail > 0 && bounce + 1 >= tune.tail && bounce + 1 < max_bounces &&
-                            npx <= (two_in_flight || cache ? SHADOW_TAIL_PX2 : SHADOW_TAIL_PX1) && !(ins && ins->counters);
+                            shadows_to_tail(npx, two_in_flight, cache != nullptr) && !(ins && ins->counters);
         const bool time_shade = ins && bounce == 0;
         if (time_shade) (void)hipEventRecord(ins->xbegin[WF_X_SHADE0], s);
         hipLaunchKernelGGL(k_shade, dim3(gblocks), dim3(WF_BLOCK), 0, s, S, fc, W, parity, shade_q, cb, cf,
