@@ -161,7 +161,7 @@ struct TraceTuning {
 constexpr int WF_MAX_TRACE_LAUNCHES = 40;
 // Further timed stages of a frame: the primary vertex's shade launch, the
 // sky pass of the tail's escaped paths, the radiance cache's inference and
-// its training steps (train, partial sums, Adam).
+// its training steps (train, Adam).
 enum { WF_X_SHADE0 = 0, WF_X_SKY = 1, WF_X_INFER = 2, WF_X_TRAIN = 3, WF_XSTAGES = 4 };
 struct WfInstrument {
     hipEvent_t begin[WF_MAX_TRACE_LAUNCHES];

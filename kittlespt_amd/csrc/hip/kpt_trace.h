@@ -34,21 +34,23 @@
 //     NodePair, so an interior step is one 64-byte line and nothing is decoded.
 //
 // What bounds it and what that decided (1000 instances, 1.24 M triangles,
-// 1920x1080 camera rays and their bounces).  The kernels issue vector
-// instructions for about three quarters of their cycles, and with 18 (camera
-// rays) or 9 (paths) of 64 lanes at work each, because a wave's lanes hold
-// different kinds of steps; the rest is waiting for the next node.  So a wave
-// runs one kind of step at a time (Trav::round), and the triangles of its
-// leaves are spread over all its lanes (Trav::leaves), half of a ray's work
-// and the half whose lanes were fewest.  Waiting for more lanes to reach the
-// chosen kind costs more than it fills: passes at 8, 4, 2 and 1 lanes at
-// leaves and instances took 1458, 1260, 1204 and 1125 us for a million
-// incoherent rays.  Interior steps come four to a round (a round of one:
-// 1590 us against 1458 for two, 1173 for four at two lanes).  Node pairs
-// instead of two-level 192-byte records: a third of the footprint and of the
-// cache accesses, and 64 registers instead of 96 (8 waves per SIMD instead of
-// 5).  Closest-hit launch 2.40 -> 1.51 ms, a million incoherent rays
-// 2.08 -> 1.10 ms, fifty thousand any-hit rays 124 -> 70 us.
+// 1920x1080 camera rays and their bounces).  With one loop in which each lane
+// ran its own kind of step, a vector instruction had 18 (camera rays) or 9
+// (paths) of 64 lanes at work.  So a wave runs one kind of step at a time
+// (Trav::round), and the triangles of its leaves are spread over all its lanes
+// (Trav::leaves), half of a ray's work and the half whose lanes were fewest.
+// Now 44 (camera rays) and 32 (paths) lanes are, and the camera rays take 0.68
+// of the instructions; at four cycles each they fill 0.8 of the SIMDs' cycles,
+// while a wave waits for 60 % of its own: instructions and latency together.
+// Waiting for more lanes to reach the chosen kind costs more than it fills:
+// passes at 8, 4, 2 and 1 lanes at leaves and instances took 1458, 1260, 1204
+// and 1125 us for a million incoherent rays.  Interior steps come four to a
+// round (a round of one: 1590 us against 1458 for two, 1173 for four at two
+// lanes).  Node pairs instead of two-level 192-byte records: a third of the
+// footprint and of the cache accesses, and 64 registers instead of 96 (8 waves
+// per SIMD instead of 5; a few more spilled cost up to twice the time).
+// Closest-hit launch alone on the GPU 2.60 -> 1.74 ms, a million incoherent
+// rays 2.09 -> 1.11 ms, fifty thousand any-hit rays 124 -> 70 us.
 // Traversal is a state machine (init / round) so persistent kernels can refill
 // a lane with a new ray, and park a lane's, between rounds.
 #pragma once
@@ -473,7 +475,8 @@ struct Trav {
     // few lanes were at one together: 200,000 rays through leaves of 9000
     // triangles ran 9.0e9 vector instructions with 12.6 lanes at work, so 2.1e9
     // with 64.  Through leaves of 160, 890 and 21,900: 970 -> 344, 6000 -> 1190
-    // and 201,200 -> 66,600 us.
+    // and 201,200 -> 66,600 us.  Kernels that meet none are up to 1 % slower for
+    // its registers (64 views 226.0 -> 227.7 ms).
     template <bool COUNT>
     __device__ __forceinline__ void wide_leaf(const SceneView& S, TraceCounts* cnt, int k) {
         const bool mine = (int)__lane_id() == k;

@@ -23,7 +23,7 @@ namespace {
 constexpr int WF_BLOCK = 256;
 // Occupancy targets in waves per SIMD (512 VGPRs per lane per SIMD): the
 // traversal kernels at 8 (64 VGPRs; the closest-hit launch of a 1080p frame
-// 1.54 ms, 1.62 at 6 waves), the path-per-lane tail at 6 (80 VGPRs, the path's
+// 5 % faster than at 6 waves), the path-per-lane tail at 6 (80 VGPRs, the path's
 // state spilled around its rounds: 64 views 229 ms, 238 at 5 waves, 257 at 4,
 // 247 at 7 and 350 at 8).
 #define KPT_WPE_TRACE __attribute__((amdgpu_waves_per_eu(8)))
